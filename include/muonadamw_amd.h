@@ -235,6 +235,26 @@ int mamw_muon_step_amp(const mamw_muon_matrix* mats, int batch, double lr,
                        const float* grad_scale, const float* found_inf,
                        mamw_stream_t stream);
 
+/* The same step on the direct path, for small launches: up to
+ * MAMW_MUON_DIRECT_MAX matrices of any shapes in one set of 2 + 3*ns_steps
+ * launches, the GEMM operands read straight into registers by one wavefront per
+ * output tile (muon_direct.hip).  Results, bit for bit, are those of
+ * mamw_muon_step / mamw_muon_step_amp on each matrix; grad_scale and found_inf
+ * as there (NULL: a plain step).  ns_steps >= 1; a matrix padded to multiples
+ * of 64 holds at most 2^26 elements (MAMW_ERR_SHAPE beyond).  The workspace
+ * (256-byte aligned, mamw_muon_direct_workspace_bytes, which reads the rows
+ * and cols only) also keeps X beside its transpose, so it is larger than
+ * mamw_muon_workspace_bytes.                                                 */
+#define MAMW_MUON_DIRECT_MAX 64
+int mamw_muon_direct_workspace_bytes(const mamw_muon_matrix* mats, int count,
+                                     int ns_steps, size_t* bytes);
+int mamw_muon_direct_step(const mamw_muon_matrix* mats, int count, double lr,
+                          double weight_decay, double beta, int nesterov,
+                          float a, float b, float c, int ns_steps, float eps,
+                          void* workspace, size_t workspace_bytes,
+                          const float* grad_scale, const float* found_inf,
+                          mamw_stream_t stream);
+
 /* ==== Newton-Schulz building blocks (batched, bf16, fp32 accumulate) ======== *
  * Operate on `batch` contiguous zero-padded row-major matrices.  m and n must
  * be multiples of 128 and k a multiple of 64; the Python mirrors pad.  An
@@ -274,7 +294,8 @@ int mamw_transpose_bf16(const uint16_t* src, uint16_t* dst, int batch,
  * runs under HIP graph capture.                                               */
 typedef struct mamw_prof_record {
     int32_t kernel;  /* see mamw_prof_kernel_name                                  */
-    int32_t variant; /* GEMMs: 8*tile + 4*(A lower-triangle) + 2*(k-major) + (k-blocked) */
+    int32_t variant; /* GEMMs: 8*tile + 4*(A lower-triangle) + 2*(k-major) + (k-blocked);
+                        direct GEMMs: 8 * edge of the square whose tiles are consecutive   */
     double  flops;   /* algorithmic floating-point operations of the launch (0: n/a) */
     double  bytes;   /* algorithmic HBM bytes of the launch (0: not known here)      */
     float   ms;      /* dispatch duration                                            */

@@ -1,0 +1,191 @@
+"""The direct path of the Muon step (csrc/muon_direct.hip): on the GPU bit for
+bit against mamw_muon_step on each matrix alone, at the edges of its tiles,
+fragments and prep units; on the CPU its argument checks, the choice between
+the two paths and the merging of launch groups.
+
+No tolerance: every output element sums the same products in the same order
+under either path (one chain of 32x32x16 MFMAs, k ascending), and the epilogues
+round at the same places."""
+
+import ctypes
+
+import pytest
+import torch
+
+from triton_muon_adamw import _lib
+from triton_muon_adamw.muon import hip_muon
+from triton_muon_adamw.muon.hip_muon import scaled_lr
+
+COEFFS = (3.4445, -4.7750, 2.0315)
+F32, BF16 = torch.float32, torch.bfloat16
+
+
+def _arr(mats):
+    arr = (_lib.MuonMatrix * len(mats))()
+    for i, (p, g, m, u) in enumerate(mats):
+        flags = (_lib.BF16_PARAM if p.dtype == BF16 else 0) | (_lib.BF16_GRAD if g.dtype == BF16 else 0)
+        arr[i] = _lib.MuonMatrix(p.data_ptr(), g.data_ptr(), m.data_ptr(), u.data_ptr() if u is not None else None,
+                                 *p.shape, scaled_lr(2e-2, "original", *p.shape), flags)
+    return arr
+
+
+def _make(shapes, dev, pd, gd, shift, with_update):
+    """[param, grad, momentum, update] per shape; `shift`: each starts one element past an aligned address."""
+    gen = torch.Generator(device=dev).manual_seed(21)
+    out = []
+    for r, c in shapes:
+        def t(std, dtype):
+            flat = torch.empty(r * c + shift, device=dev).normal_(0.0, std, generator=gen).to(dtype)
+            return flat[shift:].view(r, c)
+        out.append([t(0.02, pd), t(1e-3, gd), t(1e-3, F32), torch.zeros((r, c), device=dev) if with_update else None])
+    return out
+
+
+# one fragment and less; 32- and 64-wide edges; several prep units, ragged; all
+# in one launch, tall and wide mixed; one shape (addresses from the block
+# number); enough 64-wide tiles for the wide tile on the updates (18 x 24 = 432)
+# and on every product (32 x 33 / 2 = 528)
+SETS = [
+    [(1, 5), (5, 1), (1, 1), (31, 33), (32, 64), (33, 65), (64, 63), (65, 128), (129, 127)],
+    [(10, 517), (517, 1003), (1003, 785)],
+    [(256, 512)] * 3,
+    [(512, 256), (256, 512)],
+    [(1100, 1500)],
+    [(2048, 2000)],
+    [(192, 448)] * 33 + [(448, 192)] * 31,  # a full table
+]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shapes", SETS, ids=lambda s: f"{len(s)}x{s[0][0]}x{s[0][1]}")
+@pytest.mark.parametrize("pd,gd,shift,ns_steps,nesterov", [(F32, F32, 0, 5, 1), (BF16, BF16, 0, 2, 1),
+                                                           (F32, BF16, 1, 1, 0), (BF16, F32, 1, 3, 1)])
+def test_direct_equals_staged(gpu, shapes, pd, gd, shift, ns_steps, nesterov):
+    lib = _lib.load()
+    stream = torch.cuda.current_stream(gpu).cuda_stream
+    hyper = (2e-2, 0.1, 0.95, nesterov, *COEFFS, ns_steps, 1e-7)
+    mine, ref = (_make(shapes, gpu, pd, gd, shift, ns_steps != 2) for _ in range(2))
+    arr = _arr(mine)
+    nbytes = hip_muon._direct_workspace_bytes(arr, len(shapes), ns_steps)
+    ws = torch.full((nbytes,), 0xFF, dtype=torch.uint8, device=gpu)  # NaN wherever it is read unwritten
+    _lib.check(lib.mamw_muon_direct_step(arr, len(shapes), *hyper, ws.data_ptr(), nbytes, None, None, stream), "direct")
+    for x in ref:
+        n = hip_muon._workspace_bytes(1, *x[0].shape, ns_steps)
+        w1 = torch.empty(n, dtype=torch.uint8, device=gpu)
+        _lib.check(lib.mamw_muon_step(_arr([x]), 1, *hyper, w1.data_ptr(), n, stream), "staged")
+    torch.cuda.synchronize()
+    for i, (a, b) in enumerate(zip(mine, ref)):
+        for k, what in ((0, "param"), (2, "momentum"), (3, "update")):
+            if a[k] is not None:
+                assert torch.equal(a[k], b[k]), (i, shapes[i], what)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("inf", [0.0, 1.0])
+def test_direct_gradient_scaler_step(gpu, inf):
+    """grad_scale divides the gradients; a non-zero found_inf leaves everything as it was."""
+    lib = _lib.load()
+    stream = torch.cuda.current_stream(gpu).cuda_stream
+    hyper = (2e-2, 0.1, 0.95, 1, *COEFFS, 5, 1e-7)
+    shapes = [(100, 300), (300, 100), (64, 64)]
+    mine, ref, start = (_make(shapes, gpu, F32, F32, 0, True) for _ in range(3))
+    scale, found = torch.full((), 3.0, device=gpu), torch.full((), inf, device=gpu)
+    arr = _arr(mine)
+    nbytes = hip_muon._direct_workspace_bytes(arr, 3, 5)
+    ws = torch.empty(nbytes, dtype=torch.uint8, device=gpu)
+    _lib.check(lib.mamw_muon_direct_step(arr, 3, *hyper, ws.data_ptr(), nbytes, scale.data_ptr(), found.data_ptr(),
+                                         stream), "direct")
+    for x in ref:
+        n = hip_muon._workspace_bytes(1, *x[0].shape, 5)
+        w1 = torch.empty(n, dtype=torch.uint8, device=gpu)
+        _lib.check(lib.mamw_muon_step_amp(_arr([x]), 1, *hyper, w1.data_ptr(), n, scale.data_ptr(), found.data_ptr(),
+                                          stream), "staged")
+    torch.cuda.synchronize()
+    for a, b, s in zip(mine, ref, start):
+        for k in (0, 2, 3):
+            assert torch.equal(a[k], b[k])
+            assert torch.equal(a[k], s[k]) == (inf != 0.0)
+
+
+def _mats(specs):
+    arr = (_lib.MuonMatrix * len(specs))()
+    for i, (r, c) in enumerate(specs):
+        base = (i + 1) << 36
+        arr[i] = _lib.MuonMatrix(base, base + (1 << 34), base + (2 << 34), None, r, c, 1e-3, 0)
+    return arr
+
+
+def _bytes(arr, n, steps=5):
+    b = ctypes.c_size_t()
+    return _lib.load().mamw_muon_direct_workspace_bytes(arr, n, steps, ctypes.byref(b)), b.value
+
+
+def _step(arr, n, ws=1 << 45, ws_bytes=1 << 40, steps=5):
+    return _lib.load().mamw_muon_direct_step(arr, n, 1e-3, 0.1, 0.95, 1, *COEFFS, steps, 1e-7, ws, ws_bytes, None,
+                                             None, None)
+
+
+def test_direct_rejects_before_hip():
+    NULL, COUNT, SHAPE, ALIGN, WS, HYPER, ALIAS = -1, -2, -4, -5, -6, -7, -9
+    ok = [(10, 517), (517, 1003)]
+    st, need = _bytes(_mats(ok), 2)
+    # the table, then X^T twice and X, A and B, the unit sums, per matrix
+    rup = lambda x, t: -(-x // t) * t  # noqa: E731
+    expect = 64 * 64
+    for r, c in ok:
+        mp, np_ = rup(min(r, c), 64), rup(max(r, c), 64)
+        expect += rup(6 * mp * np_ + 4 * mp * mp + 4 * (rup(r, 128) // 32) * (rup(c, 128) // 128), 256)
+    assert (st, need) == (0, expect)
+    assert _bytes(_mats(ok), 0)[0] == COUNT and _bytes(_mats([(4, 4)] * 65), 65)[0] == COUNT
+    assert _bytes(_mats(ok), 2, steps=0)[0] == HYPER and _bytes(_mats(ok), 2, steps=100)[0] == HYPER
+    assert _bytes(_mats([(0, 4)]), 1)[0] == SHAPE and _bytes(_mats([(8192, 8256)]), 1)[0] == SHAPE
+    assert _bytes(_mats([(1, 1 << 20)]), 1)[0] == SHAPE  # too many prep units for one block to sum
+    assert _step(_mats(ok), 2, ws_bytes=need - 1) == WS and _step(_mats(ok), 2, ws=None) == WS
+    assert _step(_mats(ok), 2, ws=(1 << 45) + 64) == WS
+    for field, value, code in (("param", None, NULL), ("flags", 4, HYPER), ("momentum", (1 << 45) + 256, ALIAS),
+                               ("grad", (2 << 36) + 2, ALIGN), ("param", 1 << 36, ALIAS)):
+        arr = _mats(ok)
+        setattr(arr[1], field, value)
+        assert _step(arr, 2) == code, field
+
+
+def test_direct_choice():
+    """Small groups go direct, groups that fill the GPU with staged tiles do not; a set of classes goes as one."""
+    pays = hip_muon.direct_pays
+    for shape, count in (((512, 2048), 2), ((3072, 768), 1), ((10, 517), 32), ((2048, 2048), 1), ((1024, 4096), 1)):
+        assert pays(*shape, count, 256, 5), (shape, count)
+    for shape, count in (((512, 2048), 16), ((768, 3072), 12), ((1024, 2048), 8), ((4096, 4096), 1),
+                         ((14336, 4096), 1), ((8192, 8256), 1)):
+        assert not pays(*shape, count, 256, 5), (shape, count)
+    assert not pays(64, 64, 1, 256, 0)  # ns_steps = 0 has no product to run
+    both = hip_muon.direct_set_pays
+    assert both(((785, 1003, 1), (517, 1003, 1), (10, 517, 1)), 256, 5)
+    assert both(((256, 1024, 4), (256, 768, 2), (256, 256, 2)), 256, 5)
+    assert not both(((768, 3072, 24), (768, 2304, 12), (768, 768, 12)), 256, 5)
+    assert not both(((1024, 2048, 1), (2048, 4096, 1), (4096, 4096, 1), (1024, 4096, 1)), 256, 5)
+
+
+def test_merged_launches():
+    """Groups go out together up to the table's size and only where no matrix
+    writes what another reads or writes."""
+    def call(specs, group, first):
+        arr = (_lib.MuonMatrix * len(specs))()
+        for i, (r, c) in enumerate(specs):
+            base = (first + i + 1) << 36
+            arr[i] = _lib.MuonMatrix(base, base + (1 << 34), base + (2 << 34), None, r, c, 1e-3, 0)
+        return hip_muon._Call("d0", arr, len(specs), 0, 8, 16, group, True)
+
+    runs = lambda calls: [[c.group for c in r] for r in hip_muon._merge(calls)]  # noqa: E731
+    a, b, c = call([(8, 16)] * 30, 0, 0), call([(16, 32)] * 30, 1, 30), call([(4, 4)] * 5, 2, 60)
+    assert runs([a, b, c]) == [[0, 1], [2]]
+    a, b = call([(8, 16)], 0, 0), call([(16, 32)], 1, 1)
+    assert runs([a, b]) == [[0, 1]]
+    b.arr[0].grad = a.arr[0].grad  # two readers
+    assert runs([a, b]) == [[0, 1]]
+    b.arr[0].grad = a.arr[0].param  # one matrix's gradient is the other's parameter
+    assert runs([a, b]) == [[0], [1]]
+    b = call([(16, 32)], 1, 1)
+    b.arr[0].param = a.arr[0].param + 8 * 16 * 4 - 4  # the last element shared
+    assert runs([a, b]) == [[0], [1]]
+    b.arr[0].param += 4
+    assert runs([a, b]) == [[0, 1]]

@@ -28,6 +28,12 @@ enum KernelId : int32_t {
     K_NS_APPLY,
     K_TRANSPOSE,
     K_ADAMW_BIAS,
+    K_DIRECT_PREP,
+    K_DIRECT_SCALE,
+    K_DIRECT_GRAM,
+    K_DIRECT_POLY,
+    K_DIRECT_UPDATE,
+    K_DIRECT_APPLY,
     K_COUNT
 };
 

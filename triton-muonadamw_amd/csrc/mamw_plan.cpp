@@ -221,6 +221,48 @@ int muon_plan(int batch, int64_t rows, int64_t cols, int ns_steps, MuonPlan* pla
     return MAMW_OK;
 }
 
+// Buffers of entry i of a launch: alignment, and no overlap of memory the entry
+// writes with anything it or an earlier entry reads or writes, or with the
+// workspace.
+int muon_check_entry(const mamw_muon_matrix* mats, int i, const void* workspace, size_t workspace_bytes) {
+    const mamw_muon_matrix& M = mats[i];
+    if (!M.param || !M.grad || !M.momentum) return MAMW_ERR_NULL;
+    const size_t ep = (M.flags & MAMW_BF16_PARAM) ? 2 : 4, eg = (M.flags & MAMW_BF16_GRAD) ? 2 : 4;
+    if (!aligned(M.param, ep) || !aligned(M.grad, eg) || !aligned(M.momentum, 4)) return MAMW_ERR_ALIGN;
+    const size_t ne = size_t(M.rows) * size_t(M.cols);
+    const size_t nb = ne * 4, np_ = ne * ep, ng = ne * eg;
+    if (overlap(M.param, np_, M.grad, ng) || overlap(M.param, np_, M.momentum, nb) ||
+        overlap(M.momentum, nb, M.grad, ng))
+        return MAMW_ERR_ALIAS;
+    if (overlap(M.param, np_, workspace, workspace_bytes) || overlap(M.momentum, nb, workspace, workspace_bytes) ||
+        overlap(M.grad, ng, workspace, workspace_bytes))
+        return MAMW_ERR_ALIAS;
+    if (M.update) {
+        if (!aligned(M.update, 4)) return MAMW_ERR_ALIGN;
+        if (overlap(M.update, nb, M.param, np_) || overlap(M.update, nb, M.grad, ng) ||
+            overlap(M.update, nb, M.momentum, nb) || overlap(M.update, nb, workspace, workspace_bytes))
+            return MAMW_ERR_ALIAS;
+    }
+    // Across entries: memory one entry writes (parameter, momentum,
+    // update) must not overlap anything another entry reads or writes
+    // (the batch's kernels run over all entries at once).
+    const void* wi[3] = {M.param, M.momentum, M.update};
+    const size_t wbi[3] = {np_, nb, M.update ? nb : 0};
+    for (int j = 0; j < i; ++j) {
+        const mamw_muon_matrix& N = mats[j];
+        const size_t nej = size_t(N.rows) * size_t(N.cols);
+        const void* wj[3] = {N.param, N.momentum, N.update};
+        const size_t wbj[3] = {nej * ((N.flags & MAMW_BF16_PARAM) ? 2 : 4), nej * 4, N.update ? nej * 4 : 0};
+        const size_t ngj = nej * ((N.flags & MAMW_BF16_GRAD) ? 2 : 4);
+        for (int x = 0; x < 3; ++x) {
+            if (overlap(wi[x], wbi[x], N.grad, ngj) || overlap(wj[x], wbj[x], M.grad, ng)) return MAMW_ERR_ALIAS;
+            for (int y = 0; y < 3; ++y)
+                if (overlap(wi[x], wbi[x], wj[y], wbj[y])) return MAMW_ERR_ALIAS;
+        }
+    }
+    return MAMW_OK;
+}
+
 int muon_validate(const mamw_muon_matrix* mats, int batch, int ns_steps, const void* workspace,
                   size_t workspace_bytes, MuonPlan* plan, MuonBatchDescs* descs) {
     if (!mats || !plan || !descs) return MAMW_ERR_NULL;
@@ -237,40 +279,8 @@ int muon_validate(const mamw_muon_matrix* mats, int batch, int ns_steps, const v
         const int64_t mi = M.rows < M.cols ? M.rows : M.cols;
         const int64_t ni = M.rows < M.cols ? M.cols : M.rows;
         if (mi != plan->m || ni != plan->n) return MAMW_ERR_SHAPE;
-        if (!M.param || !M.grad || !M.momentum) return MAMW_ERR_NULL;
-        const size_t ep = (M.flags & MAMW_BF16_PARAM) ? 2 : 4, eg = (M.flags & MAMW_BF16_GRAD) ? 2 : 4;
-        if (!aligned(M.param, ep) || !aligned(M.grad, eg) || !aligned(M.momentum, 4)) return MAMW_ERR_ALIGN;
-        const size_t ne = size_t(M.rows) * size_t(M.cols);
-        const size_t nb = ne * 4, np_ = ne * ep, ng = ne * eg;
-        if (overlap(M.param, np_, M.grad, ng) || overlap(M.param, np_, M.momentum, nb) ||
-            overlap(M.momentum, nb, M.grad, ng))
-            return MAMW_ERR_ALIAS;
-        if (overlap(M.param, np_, workspace, plan->bytes) || overlap(M.momentum, nb, workspace, plan->bytes) ||
-            overlap(M.grad, ng, workspace, plan->bytes))
-            return MAMW_ERR_ALIAS;
-        if (M.update) {
-            if (!aligned(M.update, 4)) return MAMW_ERR_ALIGN;
-            if (overlap(M.update, nb, M.param, np_) || overlap(M.update, nb, M.grad, ng) ||
-                overlap(M.update, nb, M.momentum, nb) || overlap(M.update, nb, workspace, plan->bytes))
-                return MAMW_ERR_ALIAS;
-        }
-        // Across entries: memory one entry writes (parameter, momentum,
-        // update) must not overlap anything another entry reads or writes
-        // (the batch's kernels run over all entries at once).
-        const void* wi[3] = {M.param, M.momentum, M.update};
-        const size_t wbi[3] = {np_, nb, M.update ? nb : 0};
-        for (int j = 0; j < i; ++j) {
-            const mamw_muon_matrix& N = mats[j];
-            const size_t nej = size_t(N.rows) * size_t(N.cols);
-            const void* wj[3] = {N.param, N.momentum, N.update};
-            const size_t wbj[3] = {nej * ((N.flags & MAMW_BF16_PARAM) ? 2 : 4), nej * 4, N.update ? nej * 4 : 0};
-            const size_t ngj = nej * ((N.flags & MAMW_BF16_GRAD) ? 2 : 4);
-            for (int x = 0; x < 3; ++x) {
-                if (overlap(wi[x], wbi[x], N.grad, ngj) || overlap(wj[x], wbj[x], M.grad, ng)) return MAMW_ERR_ALIAS;
-                for (int y = 0; y < 3; ++y)
-                    if (overlap(wi[x], wbi[x], wj[y], wbj[y])) return MAMW_ERR_ALIAS;
-            }
-        }
+        st = muon_check_entry(mats, i, workspace, plan->bytes);
+        if (st != MAMW_OK) return st;
         MuonMatDesc& d = descs->d[i];
         d.param = M.param;
         d.grad = M.grad;
@@ -281,6 +291,63 @@ int muon_validate(const mamw_muon_matrix* mats, int batch, int ns_steps, const v
         d.slr = M.scaled_lr;
         d.tall = M.rows > M.cols ? 1 : 0;
         d.flags = M.flags;
+    }
+    return MAMW_OK;
+}
+
+// ---------------------------------------------------------------------------
+// Direct path
+
+int direct_workspace(const mamw_muon_matrix* mats, int count, int ns_steps, size_t* bytes) {
+    if (count < 1 || count > MAMW_MUON_DIRECT_MAX) return MAMW_ERR_COUNT;
+    if (ns_steps < 1 || ns_steps >= 100) return MAMW_ERR_HYPER;
+    int64_t off = int64_t(kDirectTableBytes);
+    for (int i = 0; i < count; ++i) {
+        const int64_t R = mats[i].rows, C = mats[i].cols;
+        if (R < 1 || C < 1 || R > kMaxDim || C > kMaxDim) return MAMW_ERR_SHAPE;
+        const int64_t mp = round_up(std::min(R, C), kDirectPad), np = round_up(std::max(R, C), kDirectPad);
+        if (mp * np > kDirectMaxElems) return MAMW_ERR_SHAPE;
+        const int64_t units = direct_units(int(R), int(C));
+        if (units > kDirectMaxUnits) return MAMW_ERR_SHAPE;
+        off += int64_t(align_ws(size_t(direct_off_part(mp, np) + units * 4)));
+    }
+    *bytes = size_t(off);
+    return MAMW_OK;
+}
+
+int direct_validate(const mamw_muon_matrix* mats, int count, int ns_steps, const void* workspace,
+                    size_t workspace_bytes, DirectBatch* batch) {
+    if (!mats || !batch) return MAMW_ERR_NULL;
+    size_t need = 0;
+    int st = direct_workspace(mats, count, ns_steps, &need);
+    if (st != MAMW_OK) return st;
+    if (!workspace || !aligned(workspace, kWsAlign) || workspace_bytes < need) return MAMW_ERR_WORKSPACE;
+    memset(batch, 0, sizeof(*batch));
+    batch->count = count;
+    batch->uniform = 1;
+    int64_t off = int64_t(kDirectTableBytes);
+    for (int i = 0; i < count; ++i) {
+        const mamw_muon_matrix& M = mats[i];
+        if (M.flags & ~(MAMW_BF16_PARAM | MAMW_BF16_GRAD)) return MAMW_ERR_HYPER;
+        st = muon_check_entry(mats, i, workspace, need);
+        if (st != MAMW_OK) return st;
+        DirectMat& d = batch->d[i];
+        d.param = M.param;
+        d.grad = M.grad;
+        d.mom = M.momentum;
+        d.upd = M.update;
+        d.rows = int32_t(M.rows);
+        d.cols = int32_t(M.cols);
+        d.mp = int32_t(round_up(std::min(M.rows, M.cols), kDirectPad));
+        d.np = int32_t(round_up(std::max(M.rows, M.cols), kDirectPad));
+        if (d.mp != batch->d[0].mp || d.np != batch->d[0].np ||
+            direct_units(d.rows, d.cols) != direct_units(batch->d[0].rows, batch->d[0].cols))
+            batch->uniform = 0;  // regions are then not equally spaced either
+        d.slr = M.scaled_lr;
+        d.tall = M.rows > M.cols ? 1 : 0;
+        d.flags = M.flags;
+        d.ws = uint32_t(off / int64_t(kWsAlign));
+        off += int64_t(align_ws(size_t(direct_off_part(d.mp, d.np) + direct_units(d.rows, d.cols) * 4)));
     }
     return MAMW_OK;
 }

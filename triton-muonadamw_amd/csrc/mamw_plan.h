@@ -97,6 +97,58 @@ int muon_validate(const mamw_muon_matrix* mats, int batch, int ns_steps,
                   const void* workspace, size_t workspace_bytes, MuonPlan* plan,
                   MuonBatchDescs* descs);
 
+// ---------------------------------------------------------------------------
+// Direct path (muon_direct.hip): up to MAMW_MUON_DIRECT_MAX matrices of any
+// shapes in one set of launches.  The workspace starts with the launch table
+// (a DirectMat per matrix, written by the prep kernel for those after it);
+// then each matrix has its own region, padded to multiples of 64,
+// fragment-major:
+//   X^T0 [np][mp], X [mp][np] (adjacent: the scale kernel runs over both),
+//   X^T1 [np][mp], A [mp][mp], B [mp][mp], the prep units' sums of squares.
+constexpr int kDirectPad = 64;
+constexpr int kDirectMaxUnits = 1 << 14;                 // prep units per matrix (each scale block sums them all)
+constexpr int64_t kDirectMaxElems = int64_t(1) << 26;    // padded elements per matrix (32-bit buffer offsets)
+
+constexpr int64_t direct_off_x(int64_t mp, int64_t np) { return mp * np * 2; }
+constexpr int64_t direct_off_xt1(int64_t mp, int64_t np) { return mp * np * 4; }
+constexpr int64_t direct_off_a(int64_t mp, int64_t np) { return mp * np * 6; }
+constexpr int64_t direct_off_b(int64_t mp, int64_t np) { return mp * np * 6 + mp * mp * 2; }
+constexpr int64_t direct_off_part(int64_t mp, int64_t np) { return mp * np * 6 + mp * mp * 4; }
+// Prep units of 32 x 128 elements, counted over the parameter padded to 128 x 128
+// as the LDS-staged path counts them: the same sums in the same places.
+constexpr int direct_units(int rows, int cols) { return ((rows + 127) / 128 * 4) * ((cols + 127) / 128); }
+
+struct DirectMat {
+    void* param;
+    const void* grad;
+    float* mom;
+    float* upd;  // optional orthogonalised-update output (NULL = skip)
+    int32_t rows, cols;
+    int32_t mp, np;
+    uint32_t ws;  // workspace offset of the matrix's region, in units of 256 bytes
+    float slr;
+    int32_t tall, flags;
+};
+static_assert(sizeof(DirectMat) == 64, "a launch table entry is one cache half line");
+
+constexpr size_t kDirectTableBytes = sizeof(DirectMat) * MAMW_MUON_DIRECT_MAX;
+
+// First launch block of each matrix.
+struct DirectIndex {
+    int32_t begin[MAMW_MUON_DIRECT_MAX];
+    int32_t count;
+};
+
+struct DirectBatch {
+    DirectMat d[MAMW_MUON_DIRECT_MAX];
+    int32_t count;
+    int32_t uniform;  // all matrices have one padded shape
+};
+
+int direct_workspace(const mamw_muon_matrix* mats, int count, int ns_steps, size_t* bytes);
+int direct_validate(const mamw_muon_matrix* mats, int count, int ns_steps, const void* workspace,
+                    size_t workspace_bytes, DirectBatch* batch);
+
 // Limits (documented in the ABI through the error codes).
 constexpr int64_t kMaxDim = int64_t(1) << 20;        // rows, cols <= 2^20
 constexpr int64_t kMaxMatElems = int64_t(1) << 34;   // padded m*n per matrix

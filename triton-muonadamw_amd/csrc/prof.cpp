@@ -54,7 +54,8 @@ const char* const kNames[K_COUNT] = {
     "adamw_mt_kernel", "adamw_one_kernel", "muon_prep_kernel", "muon_norm_kernel", "muon_apply0_kernel",
     "muon_scale_kernel",
     "ns_gemm_kernel:gram", "ns_gemm_kernel:poly", "ns_gemm_kernel:update", "ns_gemm_kernel:apply",
-    "transpose_bf16_kernel", "adamw_bias_kernel",
+    "transpose_bf16_kernel", "adamw_bias_kernel", "direct_prep_kernel", "direct_scale_kernel",
+    "ns_gemm_direct:gram", "ns_gemm_direct:poly", "ns_gemm_direct:update", "ns_gemm_direct:apply",
 };
 
 }  // namespace

@@ -29,7 +29,7 @@ LIB_PATH = PKG_DIR / LIB_NAME
 
 ARCH = "gfx950"
 
-SOURCES = ["mamw_plan.cpp", "abi.cpp", "prof.cpp", "adamw.hip", "muon.hip"]
+SOURCES = ["mamw_plan.cpp", "abi.cpp", "prof.cpp", "adamw.hip", "muon.hip", "muon_direct.hip"]
 
 COMMON_FLAGS = [
     "-O3",

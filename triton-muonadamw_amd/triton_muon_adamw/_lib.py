@@ -20,6 +20,7 @@ import torch
 LIB_PATH = Path(__file__).resolve().with_name("libmuonadamw_amd.so")
 ABI_VERSION = 5
 MUON_MAX_BATCH = 32
+MUON_DIRECT_MAX = 64  # MAMW_MUON_DIRECT_MAX
 BF16_PARAM = 0x1  # MAMW_BF16_PARAM
 BF16_GRAD = 0x2   # MAMW_BF16_GRAD
 
@@ -111,6 +112,12 @@ _PROTOTYPES = {
          c_int, c_float, c_void_p],
     ),
     "mamw_muon_step_amp": (
+        c_int,
+        [POINTER(MuonMatrix), c_int, c_double, c_double, c_double, c_int, c_float, c_float, c_float,
+         c_int, c_float, c_void_p, c_size_t, c_void_p, c_void_p, c_void_p],
+    ),
+    "mamw_muon_direct_workspace_bytes": (c_int, [POINTER(MuonMatrix), c_int, c_int, POINTER(c_size_t)]),
+    "mamw_muon_direct_step": (
         c_int,
         [POINTER(MuonMatrix), c_int, c_double, c_double, c_double, c_int, c_float, c_float, c_float,
          c_int, c_float, c_void_p, c_size_t, c_void_p, c_void_p, c_void_p],

@@ -31,6 +31,7 @@ normalised momentum (the reference still runs one iteration, :360).
 from __future__ import annotations
 
 import ctypes
+import functools
 import math
 import os
 from collections.abc import Iterable
@@ -66,6 +67,97 @@ def _workspace_bytes(batch: int, rows: int, cols: int, ns_steps: int) -> int:
     _lib.check(_lib.load().mamw_muon_workspace_bytes(batch, rows, cols, ns_steps, ctypes.byref(n)),
                "mamw_muon_workspace_bytes")
     return n.value
+
+
+def _direct_workspace_bytes(arr, count: int, ns_steps: int) -> int:
+    n = ctypes.c_size_t()
+    _lib.check(_lib.load().mamw_muon_direct_workspace_bytes(arr, count, ns_steps, ctypes.byref(n)),
+               "mamw_muon_direct_workspace_bytes")
+    return n.value
+
+
+# ---------------------------------------------------------------------------
+# Which kernels a launch group takes: the LDS-staged tiles (mamw_muon_step) or
+# the direct path (mamw_muon_direct_step, one wavefront per 32- or 64-wide
+# tile), the same bits either way.  Both times are estimated in microseconds
+# per step (five iterations) with constants fitted to 460 measured pairs on one
+# MI355X: 16 <= m <= 4096, n up to 16 m, 1 to 32 matrices; standard error 6%
+# each, and the cheaper path was named wrongly with a loss over 6% in 5 of
+# them.  Measured on both sides (staged / direct): 512 x 2048 one matrix 194 /
+# 101, two 198 / 116, eight 238 / 228, sixteen 328 / 374; 768 x 3072 one 268 /
+# 151, eight 438 / 518; 2048 x 2048 one 632 / 331, four 795 / 1088.
+
+def _staged_us(m: int, n: int, count: int, cus: int) -> float:
+    """Staged path: per product whole rounds of its grid (one 256-wide or two
+    128-wide workgroups per CU; a 128-wide workgroup alone on its CU is
+    faster), each a k step of 64 at 0.50 / 0.88 / 1.33 us, and 3.5 us a launch."""
+    tile = gemm_tile(m, n, count)
+    mp, np_ = _rup(m, tile), _rup(n, tile)
+    utile = 256 if (tile == 128 and m >= 1024 and mp % 256 == 0 and np_ % 256 == 0) else tile
+    tm = mp // tile
+
+    def product(t, tiles, k):
+        if t == 256:
+            rounds = -(-tiles // cus) * 1.33
+        else:
+            full, rest = divmod(tiles, 2 * cus)
+            rounds = full * 0.88 + (0.0 if rest == 0 else 0.50 if rest <= cus else 0.88)
+        return rounds * (k / 64) + 3.5
+
+    sym = count * tm * (tm + 1) // 2
+    return (5 * (product(tile, sym, np_) + product(tile, sym, mp)
+                 + product(utile, count * (mp // utile) * (np_ // utile), mp)) + 8e-6 * count * mp * np_ + 12)
+
+
+def _direct_us(groups) -> float:
+    """Direct path, one launch of all ``groups`` (m, n, count): per product 3.1
+    us, 0.035 us (32-wide) or 0.14 us (64-wide) per k step of 64 of its
+    longest reduction, and the operand bytes of all tiles at 26 TB/s (L2)."""
+    pads = [(_rup(m, 64), _rup(n, 64), count) for m, n, count in groups]
+
+    def product(tiles, k):  # tiles(mp, np, tile edge), k(mp, np)
+        wide = sum(c * tiles(mp, np_, 64) for mp, np_, c in pads) >= 384  # kDirectWideTiles
+        t = 64 if wide else 32
+        nbytes = sum(c * tiles(mp, np_, t) * 4 * t * k(mp, np_) for mp, np_, c in pads)
+        return 3.1 + max(k(mp, np_) for mp, np_, _ in pads) / 64 * (0.14 if wide else 0.035) + nbytes / 26e6
+
+    sym = lambda mp, np_, t: (mp // t) * (mp // t + 1) // 2  # noqa: E731
+    upd = lambda mp, np_, t: (mp // t) * (np_ // t)  # noqa: E731
+    return (5 * (product(sym, lambda mp, np_: np_) + product(sym, lambda mp, np_: mp)
+                 + product(upd, lambda mp, np_: mp)) + 7.6e-6 * sum(c * mp * np_ for mp, np_, c in pads) + 12)
+
+
+def _direct_fits(m: int, n: int, ns_steps: int) -> bool:
+    """The direct path's limits for one m x n (or n x m) matrix."""
+    return (ns_steps >= 1 and _rup(m, 64) * _rup(n, 64) <= 1 << 26 and _rup(m, 128) * _rup(n, 128) <= 1 << 26)
+
+
+@functools.lru_cache(maxsize=4096)
+def direct_pays(rows: int, cols: int, count: int, cus: int, ns_steps: int) -> bool:
+    """Whether a group of ``count`` rows x cols matrices, run by itself, takes
+    the direct path: where its estimate is a tenth below the staged path's (the
+    estimates' error is 6%, and the direct path's workspace is larger by X)."""
+    m, n = min(rows, cols), max(rows, cols)
+    return (_direct_fits(m, n, ns_steps)
+            and _direct_us(((m, n, count),)) < 0.9 * _staged_us(m, n, count, cus))
+
+
+@functools.lru_cache(maxsize=1024)
+def direct_set_pays(groups: tuple, cus: int, ns_steps: int) -> bool:
+    """Whether shape classes that may run beside each other (``groups``: a
+    tuple of (m, n, count)) go out as direct launches of all of them, at most
+    MUON_DIRECT_MAX matrices each, instead of staged groups on their own
+    streams: all or none, since a staged class fills the GPU and a direct one
+    beside it costs more than its staged form would (1024-2048-4096-4096-1024
+    MLP: 1748 us all staged, 2031 with its three smaller classes direct).
+    Staged classes on streams take about 1.15 times their longest class, 0.6
+    of their sum, or 95 us of host time each, whichever is most."""
+    if not all(_direct_fits(m, n, ns_steps) for m, n, _ in groups):
+        return False
+    staged = [_staged_us(m, n, count, cus) for m, n, count in groups]
+    launches = -(-sum(count for _, _, count in groups) // _lib.MUON_DIRECT_MAX)
+    direct = _direct_us(groups) + (launches - 1) * 60
+    return direct < 0.9 * max(1.15 * max(staged), 0.6 * sum(staged), 95.0 * len(groups))
 
 
 # ---------------------------------------------------------------------------
@@ -189,15 +281,18 @@ def muon_step(weights: torch.Tensor, grad: torch.Tensor, momentum: torch.Tensor,
         if out.shape != weights.shape or out.device != weights.device:
             raise ValueError("out must match the weights' shape and device")
     R, C = weights.shape
-    nbytes = _workspace_bytes(1, R, C, steps)
-    ws = torch.empty(nbytes, dtype=torch.uint8, device=weights.device)
     arr = (_lib.MuonMatrix * 1)()
     arr[0] = _lib.MuonMatrix(weights.data_ptr(), grad.data_ptr(), momentum.data_ptr(),
                              out.data_ptr() if out is not None else None, R, C, scaled_lr, 0)
     lib = _lib.load()
+    cus = torch.cuda.get_device_properties(weights.device).multi_processor_count
+    direct = direct_pays(R, C, 1, cus, steps)
+    nbytes = _direct_workspace_bytes(arr, 1, steps) if direct else _workspace_bytes(1, R, C, steps)
+    ws = torch.empty(nbytes, dtype=torch.uint8, device=weights.device)
+    args = (arr, 1, lr, weight_decay, beta, int(bool(nesterov)), a, b, c, steps, eps, ws.data_ptr(), nbytes)
     with torch.cuda.device(weights.device):
-        st = lib.mamw_muon_step(arr, 1, lr, weight_decay, beta, int(bool(nesterov)), a, b, c, steps, eps,
-                                ws.data_ptr(), nbytes, _lib.stream_handle(weights.device))
+        s = _lib.stream_handle(weights.device)
+        st = lib.mamw_muon_direct_step(*args, None, None, s) if direct else lib.mamw_muon_step(*args, s)
     _lib.check(st, "mamw_muon_step")
 
 
@@ -334,13 +429,58 @@ def _lane_split(times: list[float]) -> tuple[int, list[int]]:
 
 
 class _Call:
-    """One batched ``mamw_muon_step`` launch group (matrices of one shape class)."""
+    """One launch group (matrices of one shape class)."""
 
-    __slots__ = ("device", "arr", "n", "ws_bytes", "m", "n_", "group")
+    __slots__ = ("device", "arr", "n", "ws_bytes", "m", "n_", "group", "direct")
 
-    def __init__(self, device, arr, n, ws_bytes, m, n_, group):
+    def __init__(self, device, arr, n, ws_bytes, m, n_, group, direct=False):
         self.device, self.arr, self.n, self.ws_bytes, self.m, self.n_ = device, arr, n, ws_bytes, m, n_
         self.group = group  # index of the shape class (device, m, n)
+        self.direct = direct  # mamw_muon_direct_step (else mamw_muon_step)
+
+
+class _Launch:
+    """One library call: a launch group, or several direct-path groups together."""
+
+    __slots__ = ("device", "arr", "n", "direct", "lane", "ws_key")
+
+    def __init__(self, device, arr, n, direct, lane, ws_key):
+        self.device, self.arr, self.n, self.direct, self.lane, self.ws_key = device, arr, n, direct, lane, ws_key
+
+
+def _disjoint(calls) -> bool:
+    """Whether no memory that one matrix of ``calls`` writes (parameter,
+    momentum) is read or written by another: one launch may run them at once."""
+    spans = []
+    for c in calls:
+        for e in c.arr:
+            ne = e.rows * e.cols
+            spans.append((e.param, e.param + ne * (2 if e.flags & _lib.BF16_PARAM else 4), True))
+            spans.append((e.momentum, e.momentum + ne * 4, True))
+            spans.append((e.grad, e.grad + ne * (2 if e.flags & _lib.BF16_GRAD else 4), False))
+    spans.sort()
+    end_any = end_write = 0
+    for lo, hi, write in spans:
+        if lo < (end_any if write else end_write):
+            return False
+        end_any = max(end_any, hi)
+        if write:
+            end_write = max(end_write, hi)
+    return True
+
+
+def _merge(calls) -> list[list]:
+    """Direct-path ``calls`` as the runs that go out as one launch each: in
+    order, at most MUON_DIRECT_MAX matrices, no memory in common.  (A class's
+    later groups may hold a parameter of an earlier one again.)"""
+    runs: list[list] = []
+    for c in calls:
+        last = runs[-1] if runs else None
+        if last is not None and sum(x.n for x in last) + c.n <= _lib.MUON_DIRECT_MAX and _disjoint(last + [c]):
+            last.append(c)
+        else:
+            runs.append([c])
+    return runs
 
 
 class HipMuon:
@@ -394,9 +534,11 @@ class HipMuon:
         self._plan_key = None
         self._plan_lr = lr
         self._calls: list[_Call] = []
-        self._ws: dict = {}  # device (in order) or (device, shape class) (concurrent) -> workspace
+        self._launches: list[_Launch] = []
+        self._ws: dict = {}  # device (launches in order) or (device, shape class) (own streams) -> workspace
         self._concurrent = False
-        self._lanes: dict = {}  # (device, shape class) -> side stream, or None: the caller's stream
+        # (device, shape class) -> side stream, or None: the caller's stream (of a staged class)
+        self._lanes: dict = {}
 
     def _momentum(self, param: nn.Parameter) -> torch.Tensor:
         """The momentum buffer of ``param``, created (zero) on first use: at
@@ -428,7 +570,6 @@ class HipMuon:
         calls = []
         flops = sum(self.steps * (3.0 * m * m * n + float(m) ** 3) * len(pl) for (_, m, n), pl in groups.items())
         concurrent = len(groups) > 1 and flops <= self.concurrent_flops_limit
-        need: dict = {}
         for gi, ((dev, m, n), plist) in enumerate(groups.items()):
             one = _workspace_bytes(1, m, n, self.steps)
             limit = self.workspace_limit_bytes
@@ -455,23 +596,50 @@ class HipMuon:
                              | _lib.dtype_flag(p.grad, _lib.BF16_GRAD, "param.grad"))
                     arr[i] = _lib.MuonMatrix(p.data_ptr(), p.grad.data_ptr(), self.momentum[p].data_ptr(), None,
                                              R, C, scaled_lr(self.lr, self.adjust_lr_fn, R, C), flags)
-                wsb = _workspace_bytes(len(chunk), m, n, self.steps)
-                calls.append(_Call(dev, arr, len(chunk), wsb, m, n, gi))
-                key = (dev, gi) if concurrent else dev
+                calls.append(_Call(dev, arr, len(chunk), 0, m, n, gi))
+        # The kernels: all of a device's concurrent classes direct or none, a
+        # class that runs by itself as it pays.
+        for dev in dict.fromkeys(c.device for c in calls):
+            cus = torch.cuda.get_device_properties(dev).multi_processor_count
+            mine = [c for c in calls if c.device == dev]
+            together = concurrent and direct_set_pays(tuple((c.m, c.n_, c.n) for c in mine), cus, self.steps)
+            for c in mine:
+                c.direct = together if concurrent else direct_pays(c.m, c.n_, c.n, cus, self.steps)
+                c.ws_bytes = (_direct_workspace_bytes(c.arr, c.n, self.steps) if c.direct
+                              else _workspace_bytes(c.n, c.m, c.n_, self.steps))
+        self._lanes = {}
+        if concurrent:  # longest class first; a class's own launches keep their order (stable sort)
+            cus = {d: torch.cuda.get_device_properties(d).multi_processor_count for d in dict.fromkeys(c.device for c in calls)}
+            self._lanes, times = _lanes(calls, self.steps, cus)
+            calls.sort(key=lambda c: -times[(c.device, c.group)])
+        # The launches.  Concurrent direct classes need no streams: one launch
+        # on the caller's holds them all (up to MUON_DIRECT_MAX matrices).
+        launches, need = [], {}
+        for dev in dict.fromkeys(c.device for c in calls):
+            mine = [c for c in calls if c.device == dev]
+            for run in (_merge(mine) if concurrent and mine[0].direct else [[c] for c in mine]):
+                arr, n, wsb, lane, key = run[0].arr, run[0].n, run[0].ws_bytes, None, dev
+                if concurrent and not run[0].direct:
+                    lane, key = self._lanes[(dev, run[0].group)], (dev, run[0].group)
+                if len(run) > 1:
+                    n = sum(c.n for c in run)
+                    arr = (_lib.MuonMatrix * n)(*[e for c in run for e in c.arr])
+                    at = 0
+                    for c in run:  # the groups' entries are those of the launch
+                        c.arr = (_lib.MuonMatrix * c.n).from_buffer(arr, at * ctypes.sizeof(_lib.MuonMatrix))
+                        at += c.n
+                    wsb = _direct_workspace_bytes(arr, n, self.steps)
                 need[key] = max(need.get(key, 0), wsb)
+                launches.append(_Launch(dev, arr, n, run[0].direct, lane, key))
         for key in [k for k in self._ws if k not in need]:
             del self._ws[key]
         for key, nbytes in need.items():
             ws = self._ws.get(key)
             if ws is None or ws.numel() < nbytes:
                 self._ws[key] = None
-                self._ws[key] = torch.empty(nbytes, dtype=torch.uint8, device=key[0] if concurrent else key)
-        self._lanes = {}
-        if concurrent:  # longest class first; a class's own launches keep their order (stable sort)
-            cus = {d: torch.cuda.get_device_properties(d).multi_processor_count for d in dict.fromkeys(c.device for c in calls)}
-            self._lanes, times = _lanes(calls, self.steps, cus)
-            calls.sort(key=lambda c: -times[(c.device, c.group)])
+                self._ws[key] = torch.empty(nbytes, dtype=torch.uint8, device=key[0] if isinstance(key, tuple) else key)
         self._calls = calls
+        self._launches = launches
         self._concurrent = concurrent
 
     @torch.no_grad()
@@ -520,29 +688,29 @@ class HipMuon:
         amp = grad_scale is not None or found_inf is not None
         amp_ptrs: dict = {}  # device -> (grad_scale, found_inf) on that device, made before any fork
         if amp:
-            for call in self._calls:
+            for call in self._launches:
                 if call.device not in amp_ptrs:
                     amp_ptrs[call.device] = tuple(
                         t.to(call.device, torch.float32, non_blocking=True) if t is not None else None
                         for t in (grad_scale, found_inf))
 
         def launch(call, ws, stream_handle):
+            args = (call.arr, call.n, self.lr, self.weight_decay, self.beta, nest, self.a, self.b, self.c, self.steps,
+                    self.eps, ws.data_ptr(), ws.numel())
+            gs, fi = amp_ptrs[call.device] if amp else (None, None)
+            scaler = (gs.data_ptr() if gs is not None else None, fi.data_ptr() if fi is not None else None)
             with torch.cuda.device(call.device):
-                if not amp:
-                    st = lib.mamw_muon_step(call.arr, call.n, self.lr, self.weight_decay, self.beta, nest,
-                                            self.a, self.b, self.c, self.steps, self.eps, ws.data_ptr(),
-                                            ws.numel(), stream_handle)
+                if call.direct:
+                    st = lib.mamw_muon_direct_step(*args, *scaler, stream_handle)
+                elif not amp:
+                    st = lib.mamw_muon_step(*args, stream_handle)
                 else:
-                    gs, fi = amp_ptrs[call.device]
-                    st = lib.mamw_muon_step_amp(call.arr, call.n, self.lr, self.weight_decay, self.beta, nest,
-                                                self.a, self.b, self.c, self.steps, self.eps, ws.data_ptr(),
-                                                ws.numel(), gs.data_ptr() if gs is not None else None,
-                                                fi.data_ptr() if fi is not None else None, stream_handle)
+                    st = lib.mamw_muon_step_amp(*args, *scaler, stream_handle)
             _lib.check(st, "mamw_muon_step")
 
         if not self._concurrent:
-            for call in self._calls:
-                ws, cur = self._ws[call.device], torch.cuda.current_stream(call.device)
+            for call in self._launches:
+                ws, cur = self._ws[call.ws_key], torch.cuda.current_stream(call.device)
                 ws.record_stream(cur)  # allocated under the stream current when the plan was built
                 launch(call, ws, cur.cuda_stream)
             return
@@ -553,21 +721,20 @@ class HipMuon:
         # stream waits for all of them at the end, so the step stays ordered
         # with the caller's work on its stream.
         side = {}
-        for call in self._calls:
-            s = self._lanes[(call.device, call.group)]
+        for call in self._launches:
+            s = call.lane
             if s is not None and (call.device, id(s)) not in side:
                 side[(call.device, id(s))] = s
                 s.wait_stream(torch.cuda.current_stream(call.device))
                 for t in amp_ptrs.get(call.device, ()):  # the scaler may drop its tensors after step()
                     if t is not None:
                         t.record_stream(s)
-        for call in self._calls:
-            key = (call.device, call.group)
-            s = self._lanes[key]
+        for call in self._launches:
+            s = call.lane
             if s is None:
                 s = torch.cuda.current_stream(call.device)
-            self._ws[key].record_stream(s)
-            launch(call, self._ws[key], s.cuda_stream)
+            self._ws[call.ws_key].record_stream(s)
+            launch(call, self._ws[call.ws_key], s.cuda_stream)
         for (dev, _), s in side.items():
             torch.cuda.current_stream(dev).wait_stream(s)
 
