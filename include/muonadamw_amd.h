@@ -285,6 +285,26 @@ int mamw_ns_update(const uint16_t* B, const uint16_t* X, const uint16_t* XT,
 int mamw_transpose_bf16(const uint16_t* src, uint16_t* dst, int batch,
                         int64_t rows, int64_t cols, mamw_stream_t stream);
 
+/* The same products of one row-major bf16 matrix of any size on the direct path
+ * (no padding by the caller, 2-byte alignment): the inputs are packed into the
+ * workspace first, so out may overlap them.
+ *   MAMW_NS_GRAM    out (m x m) = X X^T            (X: m x n)
+ *   MAMW_NS_POLY    out (m x m) = b X + c X X^T    (X: m x m symmetric)
+ *   MAMW_NS_UPDATE  out (m x n) = a X + S X        (S: m x m symmetric)
+ *   MAMW_NS_STEP    out (m x n) = a X + (b A + c A A) X,  A = X X^T
+ * The same bits as mamw_ns_gram, mamw_ns_poly and mamw_ns_update.  m x n and
+ * m x m, padded to multiples of 64, hold at most 2^26 elements.  The workspace
+ * is that of (m, n); of (m, m) for MAMW_NS_POLY.                             */
+#define MAMW_NS_GRAM   0
+#define MAMW_NS_POLY   1
+#define MAMW_NS_UPDATE 2
+#define MAMW_NS_STEP   3
+int mamw_ns_direct_workspace_bytes(int64_t m, int64_t n, size_t* bytes);
+int mamw_ns_direct(int op, const uint16_t* X, const uint16_t* S, uint16_t* out,
+                   int64_t m, int64_t n, float a, float b, float c,
+                   void* workspace, size_t workspace_bytes,
+                   mamw_stream_t stream);
+
 /* ==== Profiling (opt-in) ==================================================== *
  * Between mamw_prof_start() and mamw_prof_stop(), every kernel launched by the
  * library is timed with a pair of HIP events bound to its dispatch.

@@ -189,3 +189,91 @@ def test_merged_launches():
     assert runs([a, b]) == [[0], [1]]
     b.arr[0].param += 4
     assert runs([a, b]) == [[0, 1]]
+
+
+# ---- Standalone products ----------------------------------------------------
+
+def _ns_inputs(m, n, dev):
+    gen = torch.Generator(device=dev).manual_seed(31)
+    x = (torch.empty((m, n), device=dev).normal_(generator=gen) / (m**0.5 + n**0.5)).bfloat16()
+    s = torch.empty((m, m), device=dev).normal_(generator=gen) / m
+    return x, (s + s.T).bfloat16()
+
+
+def _ns_call(op, x, s, out):
+    a, b, c = COEFFS
+    {0: lambda: hip_muon.solve_ns_kernel_1(x, out), 1: lambda: hip_muon.solve_ns_kernel_2(s, b, c, out),
+     2: lambda: hip_muon.solve_ns_kernel_3(x, s, a, out), 3: lambda: hip_muon.newton_shultz_step(x, a, b, c, out)}[op]()
+
+
+# single elements; fragment and tile edges; rows of 16-byte chunks or not; more
+# rows than columns; the 64-wide tile on the symmetric products (2048) and on
+# the update only (1280 x 1300)
+NS_SHAPES = [(1, 1), (5, 3), (31, 40), (64, 64), (65, 33), (10, 517), (517, 10), (333, 777), (128, 384), (1280, 1300),
+             (2048, 136)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape", NS_SHAPES, ids=str)
+def test_ns_direct_equals_staged(gpu, shape, monkeypatch):
+    """Bit for bit (same sums, same order), also with out over the input, which is packed first."""
+    x, s = _ns_inputs(*shape, gpu)
+    for op in range(4):
+        out = [torch.full((shape[0], shape[0]) if op < 2 else shape, 7.0, dtype=BF16, device=gpu) for _ in range(2)]
+        for o, direct in zip(out, (True, False)):
+            monkeypatch.setattr(hip_muon, "ns_direct_pays", lambda *_, d=direct: d)
+            _ns_call(op, x, s, o)
+        assert torch.equal(*out), op
+        src = s if op == 1 else x
+        if out[0].shape == src.shape:
+            own = src.clone()
+            monkeypatch.setattr(hip_muon, "ns_direct_pays", lambda *_: True)
+            _ns_call(op, own if op != 1 else x, own if op == 1 else s, own)
+            assert torch.equal(own, out[1]), op
+
+
+@pytest.mark.gpu
+def test_ns_outputs_of_any_kind(gpu):
+    """What the copy into ``out`` took, it takes: other types and strides; what it refused is refused."""
+    x, s = _ns_inputs(96, 200, gpu)
+    for op in range(4):
+        shape = (96, 96) if op < 2 else (96, 200)
+        ref = torch.empty(shape, dtype=BF16, device=gpu)
+        version = ref._version
+        _ns_call(op, x, s, ref)
+        assert ref._version > version  # an in-place write, as autograd counts them
+        wide = torch.zeros((shape[0], shape[1] + 3), dtype=BF16, device=gpu)
+        f32 = torch.empty(shape, device=gpu)
+        for o in (wide[:, 1:-2], f32, torch.empty(shape[::-1], dtype=BF16, device=gpu).T):
+            _ns_call(op, x, s, o)
+            assert torch.equal(o.to(BF16), ref), op
+        assert not wide[:, 0].any() and not wide[:, -2:].any()
+        _ns_call(op, x.T.contiguous().T, s.T.contiguous().T, f32)  # strided inputs
+        assert torch.equal(f32.to(BF16), ref)
+        leaf = torch.zeros(shape, dtype=BF16, device=gpu, requires_grad=True)
+        with pytest.raises(RuntimeError):
+            _ns_call(op, x, s, leaf)
+        with pytest.raises(RuntimeError):
+            _ns_call(op, x, s, torch.empty((shape[0], shape[1] + 1), dtype=BF16, device=gpu))
+    flat = torch.zeros(128 * 128 + 1, dtype=BF16, device=gpu)
+    with pytest.raises(ValueError):  # unpadded and misaligned
+        hip_muon.solve_ns_kernel_1(flat[1:].view(128, 128), torch.empty((128, 128), dtype=BF16, device=gpu))
+
+
+def test_ns_direct_rejects_before_hip():
+    NULL, SHAPE, ALIGN, WS, HYPER, ALIAS = -1, -4, -5, -6, -7, -9
+    lib = _lib.load()
+    n = ctypes.c_size_t()
+    assert lib.mamw_ns_direct_workspace_bytes(100, 300, ctypes.byref(n)) == 0
+    need = n.value
+    X, S, O, W = 1 << 36, 2 << 36, 3 << 36, 4 << 36
+
+    def call(op=3, x=X, s=S, o=O, m=100, k=300, ws=W, nb=need):
+        return lib.mamw_ns_direct(op, x, s, o, m, k, *COEFFS, ws, nb, None)
+
+    assert call(op=4) == HYPER and call(op=-1) == HYPER
+    assert call(m=0) == SHAPE and call(k=1 << 21) == SHAPE and call(m=8256, k=8) == SHAPE
+    assert call(x=None) == NULL and call(o=None) == NULL and call(op=2, s=None) == NULL
+    assert call(x=X + 1) == ALIGN and call(o=O + 1) == ALIGN and call(op=2, s=S + 1) == ALIGN
+    assert call(ws=None) == WS and call(ws=W + 64) == WS and call(nb=need - 1) == WS
+    assert call(x=W + 256) == ALIAS and call(o=W + 256) == ALIAS and call(op=2, s=W + 256) == ALIAS

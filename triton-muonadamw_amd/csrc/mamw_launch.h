@@ -34,6 +34,7 @@ enum KernelId : int32_t {
     K_DIRECT_POLY,
     K_DIRECT_UPDATE,
     K_DIRECT_APPLY,
+    K_DIRECT_PACK,
     K_COUNT
 };
 

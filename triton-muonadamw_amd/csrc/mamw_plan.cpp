@@ -352,4 +352,32 @@ int direct_validate(const mamw_muon_matrix* mats, int count, int ns_steps, const
     return MAMW_OK;
 }
 
+int ns_direct_plan(int64_t m, int64_t n, DirectMat* d, size_t* bytes) {
+    if (m < 1 || n < 1 || m > kMaxDim || n > kMaxDim) return MAMW_ERR_SHAPE;
+    const int64_t mp = round_up(m, kDirectPad), np = round_up(n, kDirectPad);
+    if (mp * np > kDirectMaxElems || mp * mp > kDirectMaxElems) return MAMW_ERR_SHAPE;
+    memset(d, 0, sizeof(*d));
+    d->rows = int32_t(m);
+    d->cols = int32_t(n);
+    d->mp = int32_t(mp);
+    d->np = int32_t(np);
+    d->ws = uint32_t(kDirectTableBytes / kWsAlign);
+    *bytes = align_ws(kDirectTableBytes + size_t(direct_off_part(mp, np)));
+    return MAMW_OK;
+}
+
+int ns_direct_validate(int op, const void* X, const void* S, const void* out, int64_t m, int64_t n,
+                       const void* workspace, size_t workspace_bytes, size_t need) {
+    const bool update = op == MAMW_NS_UPDATE;
+    if (!X || !out || (update && !S)) return MAMW_ERR_NULL;
+    if (!aligned(X, 2) || !aligned(out, 2) || (update && !aligned(S, 2))) return MAMW_ERR_ALIGN;
+    if (!workspace || !aligned(workspace, kWsAlign) || workspace_bytes < need) return MAMW_ERR_WORKSPACE;
+    const size_t xb = size_t(m) * size_t(op == MAMW_NS_POLY ? m : n) * 2, sb = size_t(m) * size_t(m) * 2;
+    const size_t ob = op == MAMW_NS_GRAM || op == MAMW_NS_POLY ? sb : xb;
+    if (overlap(X, xb, workspace, need) || overlap(out, ob, workspace, need) ||
+        (update && overlap(S, sb, workspace, need)))
+        return MAMW_ERR_ALIAS;
+    return MAMW_OK;
+}
+
 }  // namespace mamw

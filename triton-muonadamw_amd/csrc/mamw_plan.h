@@ -149,6 +149,12 @@ int direct_workspace(const mamw_muon_matrix* mats, int count, int ns_steps, size
 int direct_validate(const mamw_muon_matrix* mats, int count, int ns_steps, const void* workspace,
                     size_t workspace_bytes, DirectBatch* batch);
 
+// Standalone products (mamw_ns_direct) of an m x n matrix, m and n in any order:
+// the plan of its region, and the buffers.
+int ns_direct_plan(int64_t m, int64_t n, DirectMat* d, size_t* bytes);
+int ns_direct_validate(int op, const void* X, const void* S, const void* out, int64_t m, int64_t n,
+                       const void* workspace, size_t workspace_bytes, size_t need);
+
 // Limits (documented in the ABI through the error codes).
 constexpr int64_t kMaxDim = int64_t(1) << 20;        // rows, cols <= 2^20
 constexpr int64_t kMaxMatElems = int64_t(1) << 34;   // padded m*n per matrix

@@ -96,6 +96,38 @@ __device__ __forceinline__ int xcd_contiguous(int block, int total) {
     return x * q + min(x, r) + (block >> 3);
 }
 
+// A 32 x 128 tile in LDS (rows of LD halves) at (r0, c0) of an Rp x Cp matrix
+// into the fragment-major `along` (same rows) and `across` (transposed), if not
+// NULL: 8 blocks of 1 KB each, as far as the matrix goes.
+template <int LD>
+__device__ __forceinline__ void store_unit(const uint16_t* tile, int tid, int r0, int c0, int Rp, int Cp, uint16_t* along,
+                                           uint16_t* across) {
+    if (along) {
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+            const int id = tid + 256 * k, blk = id >> 6, row = id & 31, half = (id >> 5) & 1;
+            const int cc = blk * 16 + half * 8;
+            if (c0 + blk * 16 < Cp)
+                *reinterpret_cast<uint4*>(along + foff(Rp, r0 + row, c0 + cc)) =
+                    *reinterpret_cast<const uint4*>(&tile[row * LD + cc]);
+        }
+    }
+    if (across) {
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+            const int id = tid + 256 * k, blk = id >> 6, half = (id >> 5) & 1;
+            const int cl = (blk >> 1) * 32 + (id & 31), rl = (blk & 1) * 16 + half * 8;
+            if (c0 + (blk >> 1) * 32 < Cp) {
+                uint32_t w[4];
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+                    w[q] = uint32_t(tile[(rl + 2 * q) * LD + cl]) | (uint32_t(tile[(rl + 2 * q + 1) * LD + cl]) << 16);
+                *reinterpret_cast<uint4*>(across + foff(Cp, c0 + cl, r0 + rl)) = make_uint4(w[0], w[1], w[2], w[3]);
+            }
+        }
+    }
+}
+
 // ---------------------------------------------------------------------------
 // Prep: one unit of 32 x 128 parameter elements per block.  Memory-bound (14 +
 // 2 bytes per element); all of a block's loads are issued before its stores.
@@ -203,27 +235,40 @@ __global__ __launch_bounds__(256) void direct_prep_kernel(const DirectBatch b, c
     uint16_t* xm = reinterpret_cast<uint16_t*>(base + direct_off_x(d.mp, d.np));
     uint16_t* along = d.tall ? xt : xm;
     uint16_t* across = d.tall ? xm : xt;
-    if (r0 >= Rp) return;
+    if (r0 < Rp) store_unit<LD>(tile, tid, r0, c0, Rp, Cp, along, across);
+}
+
+// A row-major bf16 matrix (rows x cols) into fragment-major matrices padded
+// with zeros to Rp x Cp: `along` (its rows are rows) and, if not NULL, `across`
+// (its columns are rows).  32 x 128 elements per block.
+__global__ __launch_bounds__(256) void direct_pack_kernel(const uint16_t* __restrict__ src, int R, int C, int Rp, int Cp,
+                                                          uint16_t* __restrict__ along, uint16_t* __restrict__ across) {
+    constexpr int LD = 128 + 8;
+    __shared__ __attribute__((aligned(16))) uint16_t tile[32 * LD];
+    const int tid = threadIdx.x, pieces = (Cp + 127) >> 7;
+    const int r0 = (int(blockIdx.x) / pieces) * 32, c0 = (int(blockIdx.x) % pieces) * 128;
+    const bool vec = (C & 7) == 0 && (reinterpret_cast<uintptr_t>(src) & 15) == 0;
+    if (vec) {  // 8 columns of rows tid / 16 and + 16
+        uint4 w[2];
 #pragma unroll
-    for (int k = 0; k < 2; ++k) {
-        const int id = tid + 256 * k, blk = id >> 6, row = id & 31, half = (id >> 5) & 1;
-        const int cc = blk * 16 + half * 8;
-        if (c0 + blk * 16 < Cp)
-            *reinterpret_cast<uint4*>(along + foff(Rp, r0 + row, c0 + cc)) =
-                *reinterpret_cast<const uint4*>(&tile[row * LD + cc]);
-    }
-#pragma unroll
-    for (int k = 0; k < 2; ++k) {
-        const int id = tid + 256 * k, blk = id >> 6, half = (id >> 5) & 1;
-        const int cl = (blk >> 1) * 32 + (id & 31), rl = (blk & 1) * 16 + half * 8;
-        if (c0 + (blk >> 1) * 32 < Cp) {
-            uint32_t w[4];
-#pragma unroll
-            for (int q = 0; q < 4; ++q)
-                w[q] = uint32_t(tile[(rl + 2 * q) * LD + cl]) | (uint32_t(tile[(rl + 2 * q + 1) * LD + cl]) << 16);
-            *reinterpret_cast<uint4*>(across + foff(Cp, c0 + cl, r0 + rl)) = make_uint4(w[0], w[1], w[2], w[3]);
+        for (int p = 0; p < 2; ++p) {
+            const int r = r0 + (tid >> 4) + 16 * p, c = c0 + (tid & 15) * 8;
+            w[p] = r < R && c < C ? *reinterpret_cast<const uint4*>(src + int64_t(r) * C + c) : make_uint4(0, 0, 0, 0);
         }
+#pragma unroll
+        for (int p = 0; p < 2; ++p) *reinterpret_cast<uint4*>(&tile[((tid >> 4) + 16 * p) * LD + (tid & 15) * 8]) = w[p];
+    } else {  // single elements, 128 lanes a row
+        uint16_t h[16];
+#pragma unroll
+        for (int p = 0; p < 16; ++p) {
+            const int r = r0 + (tid >> 7) + 2 * p, c = c0 + (tid & 127);
+            h[p] = r < R && c < C ? src[int64_t(r) * C + c] : uint16_t(0);
+        }
+#pragma unroll
+        for (int p = 0; p < 16; ++p) tile[((tid >> 7) + 2 * p) * LD + (tid & 127)] = h[p];
     }
+    __syncthreads();
+    store_unit<LD>(tile, tid, r0, c0, Rp, Cp, along, across);
 }
 
 // Norm and scale: X and X^T lie one after the other, 8192 elements per block.
@@ -282,14 +327,19 @@ struct DirectGemm {
     int cur;      // which X^T buffer holds the iterate
     int super;    // tiles per edge of the square whose tiles are consecutive
     const float* found_inf;
+    uint16_t* out;  // ROWMAJOR: output, its rows and columns
+    int orows, ocols;
 };
 
-template <int MODE, int T>
+// ROWMAJOR: the product goes out as a row-major bf16 matrix (the standalone
+// functions), rows and columns beyond it dropped.
+template <int MODE, int T, bool ROWMAJOR = false>
 __global__ __launch_bounds__(64, 2) void direct_gemm_kernel(char* ws, const DirectGemm g, const DirectIndex ix) {
     constexpr bool SYM = MODE == DM_GRAM || MODE == DM_POLY;
     constexpr int F = T / 32;              // fragments per tile edge
         constexpr int D = T == 32 ? 4 : 2;     // panels of 64 k in the register ring
-    constexpr int LD = 36;                 // halves per LDS row of a 32 x 32 fragment
+    // Halves per LDS row of a 32 x 32 fragment; rows read as 16-byte chunks are aligned.
+    constexpr int LD = ROWMAJOR ? 40 : 36;
     __shared__ __attribute__((aligned(16))) uint16_t tr[32 * LD];
     if constexpr (MODE == DM_APPLY) {
         if (g.found_inf && *g.found_inf != 0.0f) return;
@@ -531,6 +581,57 @@ __global__ __launch_bounds__(64, 2) void direct_gemm_kernel(char* ws, const Dire
         return;
     }
 
+    if constexpr (ROWMAJOR) {
+        // Each fragment through LDS (tr[x][y]), then rows of 64 bytes: 4 lanes
+        // a row in 16-byte chunks where the rows allow it, else 32 lanes a row
+        // in single elements.
+        uint16_t* const out = g.out;
+        const int orows = g.orows, ocols = g.ocols;
+        const bool vec = (ocols & 7) == 0 && (reinterpret_cast<uintptr_t>(out) & 15) == 0;
+#pragma unroll
+        for (int a = 0; a < F; ++a)
+#pragma unroll
+            for (int c = 0; c < F; ++c) {
+                if (SYM && a > c && ty == tx) continue;  // the mirror of (c, a)
+                const int x0 = tx * T + c * 32, y0 = ty * T + a * 32;
+                if (a + c > 0) __syncthreads();  // the previous fragment has been read
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+                    *reinterpret_cast<uint2*>(&tr[(lane & 31) * LD + q * 8 + (lane >> 5) * 4]) = value(a, c, q);
+                __syncthreads();
+                // C[y][x]: tr[x][y], of a symmetric product's diagonal fragment
+                // the upper triangle (y <= x) for both.
+                const bool diag = SYM && x0 == y0;
+                auto at = [&](int y, int x) { return diag && y > x ? tr[y * LD + x] : tr[x * LD + y]; };
+                const bool mirror = SYM && !diag;
+                if (vec) {
+                    const int ch = (lane & 3) * 8;
+#pragma unroll
+                    for (int k = 0; k < 2; ++k) {
+                        const int r = k * 16 + (lane >> 2);
+                        uint32_t w[4];
+#pragma unroll
+                        for (int e = 0; e < 4; ++e)
+                            w[e] = uint32_t(at(r, ch + 2 * e)) | (uint32_t(at(r, ch + 2 * e + 1)) << 16);
+                        if (y0 + r < orows && x0 + ch < ocols)
+                            *reinterpret_cast<uint4*>(out + int64_t(y0 + r) * ocols + x0 + ch) = make_uint4(w[0], w[1], w[2], w[3]);
+                        if (mirror && x0 + r < orows && y0 + ch < ocols)
+                            *reinterpret_cast<uint4*>(out + int64_t(x0 + r) * ocols + y0 + ch) =
+                                *reinterpret_cast<const uint4*>(&tr[r * LD + ch]);
+                    }
+                } else {
+                    const int e = lane & 31;
+#pragma unroll
+                    for (int k = 0; k < 16; ++k) {
+                        const int r = 2 * k + (lane >> 5);
+                        if (y0 + r < orows && x0 + e < ocols) out[int64_t(y0 + r) * ocols + x0 + e] = at(r, e);
+                        if (mirror && x0 + r < orows && y0 + e < ocols) out[int64_t(x0 + r) * ocols + y0 + e] = tr[r * LD + e];
+                    }
+                }
+            }
+        return;
+    }
+
     // "Across" (rows x, 4 consecutive y per lane) needs no transpose: lanes l
     // and l + 32 fill one 16-byte chunk.  "Along" (rows y) goes through LDS,
     // one fragment at a time, and comes back by transpose reads: in a 16-lane
@@ -543,6 +644,7 @@ __global__ __launch_bounds__(64, 2) void direct_gemm_kernel(char* ws, const Dire
     for (int a = 0; a < F; ++a)
 #pragma unroll
         for (int c = 0; c < F; ++c) {
+            if (SYM && a > c && ty == tx) continue;  // the mirror of (c, a)
             const int x0 = tx * T + c * 32, y0 = ty * T + a * 32;
             const bool both = !SYM || x0 != y0;  // a diagonal fragment is its own mirror
             if (both && a + c > 0) __syncthreads();  // the previous fragment has been read
@@ -588,7 +690,7 @@ int64_t count_tiles(const DirectBatch& b, int T) {
 // 78 / 84, 2 x 512 x 2048 (512) 122 / 119, 768 x 3072 (576) 157 / 151.
 constexpr int64_t kDirectWideTiles = 384;
 
-template <int MODE>
+template <int MODE, bool ROWMAJOR = false>
 hipError_t launch_direct(const DirectBatch& b, char* ws, const DirectGemm& g, double flops, hipStream_t s) {
     const int T = count_tiles<MODE>(b, 64) >= kDirectWideTiles ? 64 : 32;
     DirectIndex x{};
@@ -616,8 +718,8 @@ hipError_t launch_direct(const DirectBatch& b, char* ws, const DirectGemm& g, do
         ga.stride = b.count > 1 ? b.d[1].ws - b.d[0].ws : 0;
     }
     const dim3 grid{unsigned(total)}, block{64};
-    if (T == 64) return launch(kid, 8 * square, flops, 0.0, direct_gemm_kernel<MODE, 64>, grid, block, s, ws, ga, x);
-    return launch(kid, 8 * square, flops, 0.0, direct_gemm_kernel<MODE, 32>, grid, block, s, ws, ga, x);
+    if (T == 64) return launch(kid, 8 * square, flops, 0.0, direct_gemm_kernel<MODE, 64, ROWMAJOR>, grid, block, s, ws, ga, x);
+    return launch(kid, 8 * square, flops, 0.0, direct_gemm_kernel<MODE, 32, ROWMAJOR>, grid, block, s, ws, ga, x);
 }
 
 }  // namespace
@@ -686,4 +788,61 @@ extern "C" int mamw_muon_direct_step(const mamw_muon_matrix* mats, int count, do
         if (e != hipSuccess) return int(e);
     }
     return MAMW_OK;
+}
+
+// ---------------------------------------------------------------------------
+// Standalone products of one row-major matrix.
+
+extern "C" int mamw_ns_direct_workspace_bytes(int64_t m, int64_t n, size_t* bytes) {
+    if (!bytes) return MAMW_ERR_NULL;
+    DirectMat d;
+    return ns_direct_plan(m, n, &d, bytes);
+}
+
+extern "C" int mamw_ns_direct(int op, const uint16_t* X, const uint16_t* S, uint16_t* out, int64_t m, int64_t n, float a,
+                              float b, float c, void* workspace, size_t workspace_bytes, mamw_stream_t stream) {
+    if (op < MAMW_NS_GRAM || op > MAMW_NS_STEP) return MAMW_ERR_HYPER;
+    DirectBatch B{};
+    size_t need = 0;
+    int st = ns_direct_plan(m, op == MAMW_NS_POLY ? m : n, &B.d[0], &need);
+    if (st != MAMW_OK) return st;
+    st = ns_direct_validate(op, X, S, out, m, n, workspace, workspace_bytes, need);
+    if (st != MAMW_OK) return st;
+    B.count = B.uniform = 1;
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    char* ws = static_cast<char*>(workspace);
+    char* base = ws + kDirectTableBytes;
+    const int mp = B.d[0].mp, np = B.d[0].np;
+    uint16_t* const xt = reinterpret_cast<uint16_t*>(base);
+    uint16_t* const x = reinterpret_cast<uint16_t*>(base + direct_off_x(mp, np));
+    uint16_t* const A = reinterpret_cast<uint16_t*>(base + direct_off_a(mp, np));
+    uint16_t* const Bm = reinterpret_cast<uint16_t*>(base + direct_off_b(mp, np));
+    auto pack = [&](const uint16_t* src, int64_t cols, int cp, uint16_t* along, uint16_t* across) {
+        return launch(K_DIRECT_PACK, 0, 0.0, double(m) * double(cols) * 2.0 * (1 + (along != nullptr) + (across != nullptr)),
+                      direct_pack_kernel, dim3(unsigned(mp / 32) * unsigned((cp + 127) / 128)), dim3(256), s, src, int(m),
+                      int(cols), mp, cp, along, across);
+    };
+    DirectGemm g{};
+    g.out = out;
+    g.orows = int(m);
+    g.ocols = int(op == MAMW_NS_GRAM || op == MAMW_NS_POLY ? m : n);
+    const double M = double(m), N = double(n);
+    hipError_t e = op == MAMW_NS_POLY ? pack(X, m, mp, A, nullptr)
+                                      : pack(X, n, np, op == MAMW_NS_UPDATE ? nullptr : x, op == MAMW_NS_GRAM ? nullptr : xt);
+    if (e == hipSuccess && op == MAMW_NS_UPDATE) e = pack(S, m, mp, Bm, nullptr);
+    if (e != hipSuccess) return int(e);
+    if (op == MAMW_NS_GRAM) return int(launch_direct<DM_GRAM, true>(B, ws, g, M * M * N, s));
+    if (op == MAMW_NS_STEP) {
+        e = launch_direct<DM_GRAM>(B, ws, g, M * M * N, s);
+        if (e != hipSuccess) return int(e);
+    }
+    g.alpha = c;
+    g.beta = b;
+    if (op == MAMW_NS_POLY) return int(launch_direct<DM_POLY, true>(B, ws, g, M * M * M, s));
+    if (op == MAMW_NS_STEP) {
+        e = launch_direct<DM_POLY>(B, ws, g, M * M * M, s);
+        if (e != hipSuccess) return int(e);
+    }
+    g.beta = a;
+    return int(launch_direct<DM_UPDATE, true>(B, ws, g, 2.0 * M * M * N, s));
 }

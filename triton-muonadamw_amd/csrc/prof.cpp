@@ -56,6 +56,7 @@ const char* const kNames[K_COUNT] = {
     "ns_gemm_kernel:gram", "ns_gemm_kernel:poly", "ns_gemm_kernel:update", "ns_gemm_kernel:apply",
     "transpose_bf16_kernel", "adamw_bias_kernel", "direct_prep_kernel", "direct_scale_kernel",
     "ns_gemm_direct:gram", "ns_gemm_direct:poly", "ns_gemm_direct:update", "ns_gemm_direct:apply",
+    "direct_pack_kernel",
 };
 
 }  // namespace

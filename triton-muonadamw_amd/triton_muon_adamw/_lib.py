@@ -129,6 +129,11 @@ _PROTOTYPES = {
         [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int64, c_int64, c_float, c_void_p],
     ),
     "mamw_transpose_bf16": (c_int, [c_void_p, c_void_p, c_int, c_int64, c_int64, c_void_p]),
+    "mamw_ns_direct_workspace_bytes": (c_int, [c_int64, c_int64, POINTER(c_size_t)]),
+    "mamw_ns_direct": (
+        c_int,
+        [c_int, c_void_p, c_void_p, c_void_p, c_int64, c_int64, c_float, c_float, c_float, c_void_p, c_size_t, c_void_p],
+    ),
     "mamw_prof_start": (c_int, []),
     "mamw_prof_stop": (c_int, []),
     "mamw_prof_collect": (c_int, [POINTER(ProfRecord), c_int, POINTER(c_int)]),

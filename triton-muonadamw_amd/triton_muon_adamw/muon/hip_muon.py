@@ -87,39 +87,46 @@ def _direct_workspace_bytes(arr, count: int, ns_steps: int) -> int:
 # 101, two 198 / 116, eight 238 / 228, sixteen 328 / 374; 768 x 3072 one 268 /
 # 151, eight 438 / 518; 2048 x 2048 one 632 / 331, four 795 / 1088.
 
-def _staged_us(m: int, n: int, count: int, cus: int) -> float:
-    """Staged path: per product whole rounds of its grid (one 256-wide or two
+def _staged_product_us(tile: int, tiles: int, k: int, cus: int) -> float:
+    """One staged product: whole rounds of its grid (one 256-wide or two
     128-wide workgroups per CU; a 128-wide workgroup alone on its CU is
-    faster), each a k step of 64 at 0.50 / 0.88 / 1.33 us, and 3.5 us a launch."""
+    faster), a k step of 64 at 1.33, 0.88 or 0.50 us, and 3.5 us a launch."""
+    if tile == 256:
+        rounds = -(-tiles // cus) * 1.33
+    else:
+        full, rest = divmod(tiles, 2 * cus)
+        rounds = full * 0.88 + (0.0 if rest == 0 else 0.50 if rest <= cus else 0.88)
+    return rounds * (k / 64) + 3.5
+
+
+def _direct_product_us(t64: int, t32: int, k: int, nbytes64: float, nbytes32: float) -> float:
+    """One direct product of ``t64`` 64-wide (or ``t32`` 32-wide) tiles: 3.1 us,
+    0.14 us (0.035 us) per k step of 64 of its longest reduction ``k``, and the
+    operand bytes of all tiles at 26 TB/s (L2)."""
+    wide = t64 >= 384  # kDirectWideTiles
+    return 3.1 + (k / 64) * (0.14 if wide else 0.035) + (nbytes64 if wide else nbytes32) / 26e6
+
+
+def _staged_us(m: int, n: int, count: int, cus: int) -> float:
+    """A step of ``count`` m x n matrices on the staged path."""
     tile = gemm_tile(m, n, count)
     mp, np_ = _rup(m, tile), _rup(n, tile)
     utile = 256 if (tile == 128 and m >= 1024 and mp % 256 == 0 and np_ % 256 == 0) else tile
     tm = mp // tile
-
-    def product(t, tiles, k):
-        if t == 256:
-            rounds = -(-tiles // cus) * 1.33
-        else:
-            full, rest = divmod(tiles, 2 * cus)
-            rounds = full * 0.88 + (0.0 if rest == 0 else 0.50 if rest <= cus else 0.88)
-        return rounds * (k / 64) + 3.5
-
     sym = count * tm * (tm + 1) // 2
-    return (5 * (product(tile, sym, np_) + product(tile, sym, mp)
-                 + product(utile, count * (mp // utile) * (np_ // utile), mp)) + 8e-6 * count * mp * np_ + 12)
+    return (5 * (_staged_product_us(tile, sym, np_, cus) + _staged_product_us(tile, sym, mp, cus)
+                 + _staged_product_us(utile, count * (mp // utile) * (np_ // utile), mp, cus))
+            + 8e-6 * count * mp * np_ + 12)
 
 
 def _direct_us(groups) -> float:
-    """Direct path, one launch of all ``groups`` (m, n, count): per product 3.1
-    us, 0.035 us (32-wide) or 0.14 us (64-wide) per k step of 64 of its
-    longest reduction, and the operand bytes of all tiles at 26 TB/s (L2)."""
+    """A step on the direct path, one launch of all ``groups`` (m, n, count)."""
     pads = [(_rup(m, 64), _rup(n, 64), count) for m, n, count in groups]
 
     def product(tiles, k):  # tiles(mp, np, tile edge), k(mp, np)
-        wide = sum(c * tiles(mp, np_, 64) for mp, np_, c in pads) >= 384  # kDirectWideTiles
-        t = 64 if wide else 32
-        nbytes = sum(c * tiles(mp, np_, t) * 4 * t * k(mp, np_) for mp, np_, c in pads)
-        return 3.1 + max(k(mp, np_) for mp, np_, _ in pads) / 64 * (0.14 if wide else 0.035) + nbytes / 26e6
+        t64, t32 = (sum(c * tiles(mp, np_, t) for mp, np_, c in pads) for t in (64, 32))
+        b64, b32 = (sum(c * tiles(mp, np_, t) * 4.0 * t * k(mp, np_) for mp, np_, c in pads) for t in (64, 32))
+        return _direct_product_us(t64, t32, max(k(mp, np_) for mp, np_, _ in pads), b64, b32)
 
     sym = lambda mp, np_, t: (mp // t) * (mp // t + 1) // 2  # noqa: E731
     upd = lambda mp, np_, t: (mp // t) * (np_ // t)  # noqa: E731
@@ -185,9 +192,82 @@ def _check_bf16_2d(x: torch.Tensor, name: str) -> None:
         raise TypeError(f"{name} must be bfloat16 (got {x.dtype})")
 
 
+_NS_GRAM, _NS_POLY, _NS_UPDATE, _NS_STEP = range(4)  # MAMW_NS_*
+
+
+@functools.lru_cache(maxsize=4096)
+def ns_direct_pays(op: int, m: int, n: int, cus: int) -> bool:
+    """Whether a standalone product takes the direct path: the estimates of its
+    products (those of the steps above), and what each path does around them:
+    packing (5 us) there; the copy into ``out``, for the update and the
+    iteration a transpose, and padding here.  Measured staged / direct, us:
+    Gram of 1024 x 4096 44 / 23, 1531 x 3001 50 / 30, 4096 x 4096 91 / 124;
+    polynomial of 1024 15 / 11, 3072 73 / 56, 4096 94 / 121; update of 768 x
+    3001 48 / 22, 2048 x 8192 90 / 105; iteration of 512 x 512 36 / 14, 1024 x
+    4096 86 / 42, 4096 x 4096 295 / 388."""
+    if max(_rup(m, 64) * _rup(n, 64), _rup(m, 64) ** 2) > 1 << 26:
+        return False
+    mp, np_ = _rup(m, 128), _rup(n, 128)
+    tile = 256 if m >= 2048 and mp % 256 == 0 else 128
+    utile = tile if np_ % 256 == 0 else 128
+    sym = (mp // tile) * (mp // tile + 1) // 2
+    d, e = _rup(m, 64), _rup(n, 64)
+    r, r2 = d // 64, d // 32
+    s64, s32 = r * (r + 1) // 2, r2 * (r2 + 1) // 2
+    u64, u32 = r * (e // 64), r2 * (e // 32)
+    products = {
+        _NS_GRAM: (_staged_product_us(tile, sym, np_, cus),
+                   _direct_product_us(s64, s32, e, s64 * 256.0 * e, s32 * 128.0 * e)),
+        _NS_POLY: (_staged_product_us(tile, sym, mp, cus),
+                   _direct_product_us(s64, s32, d, s64 * 256.0 * d, s32 * 128.0 * d)),
+        _NS_UPDATE: (_staged_product_us(utile, (mp // utile) * (np_ // utile), mp, cus),
+                     _direct_product_us(u64, u32, d, u64 * 256.0 * d, u32 * 128.0 * d)),
+    }
+    staged = direct = 5.0
+    for k in (_NS_GRAM, _NS_POLY, _NS_UPDATE) if op == _NS_STEP else (op,):
+        staged, direct = staged + products[k][0], direct + products[k][1]
+    if op >= _NS_UPDATE:
+        staged += 4 + 1.5e-6 * mp * np_
+    return direct < 0.95 * staged
+
+
+def _ns_direct(op: int, X: torch.Tensor, S, out: torch.Tensor, a: float, b: float, c: float) -> bool:
+    """The product on the direct path, straight into ``out``; False where it
+    stays with the padded, staged one: inputs or an output that are not plain
+    contiguous bf16 matrices of the right shape on one device (copies there
+    handle any strides, types and broadcasts, and refuse what autograd must
+    refuse), 16-byte misaligned inputs (which it refuses unless it pads them),
+    and sizes where it is the faster one."""
+    m, n = X.shape
+    shape = (m, m) if op in (_NS_GRAM, _NS_POLY) else (m, n)
+    if (m < 1 or n < 1 or out.dtype != torch.bfloat16 or out.shape != shape or out.device != X.device
+            or not out.is_contiguous() or out.requires_grad or out.is_inference()):
+        return False
+    for t in (X,) if S is None else (X, S):
+        if not t.is_contiguous() or t.data_ptr() % 16 or t.device != X.device:
+            return False
+    if S is not None and S.shape != (m, m) or op == _NS_POLY and n != m:
+        return False
+    dev = X.device
+    if not ns_direct_pays(op, m, n, torch.cuda.get_device_properties(dev).multi_processor_count):
+        return False
+    lib = _lib.load()
+    nbytes = ctypes.c_size_t()
+    _lib.check(lib.mamw_ns_direct_workspace_bytes(m, n, ctypes.byref(nbytes)), "mamw_ns_direct_workspace_bytes")
+    ws = torch.empty(nbytes.value, dtype=torch.uint8, device=dev)
+    with torch.cuda.device(dev):
+        st = lib.mamw_ns_direct(op, X.data_ptr(), S.data_ptr() if S is not None else None, out.data_ptr(), m, n, a, b,
+                                c, ws.data_ptr(), nbytes.value, _lib.stream_handle(dev))
+    _lib.check(st, "mamw_ns_direct")
+    torch.autograd.graph.increment_version(out)  # written in place, as copy_ records
+    return True
+
+
 def solve_ns_kernel_1(matrix: torch.Tensor, out: torch.Tensor) -> None:
     """out = matrix @ matrix.T for a bf16 m x k matrix (triton_muon.py:95-117)."""
     _check_bf16_2d(matrix, "matrix")
+    if _ns_direct(_NS_GRAM, matrix, None, out, 0.0, 0.0, 0.0):
+        return
     m, k = matrix.shape
     mp, kp = _rup(m, 128), _rup(k, 64)
     X = _padded(matrix, mp, kp)
@@ -202,6 +282,8 @@ def solve_ns_kernel_1(matrix: torch.Tensor, out: torch.Tensor) -> None:
 def solve_ns_kernel_2(matrix: torch.Tensor, b: float, c: float, out: torch.Tensor) -> None:
     """out = b*A + c*(A @ A.T) for a symmetric bf16 m x m matrix A (triton_muon.py:191-212)."""
     _check_bf16_2d(matrix, "matrix")
+    if _ns_direct(_NS_POLY, matrix, None, out, 0.0, b, c):
+        return
     m = matrix.shape[0]
     mp = _rup(m, 128)
     A = _padded(matrix, mp, mp)
@@ -227,6 +309,8 @@ def solve_ns_kernel_3(X: torch.Tensor, out_2: torch.Tensor, a: float, out: torch
     """out = a*X + out_2 @ X for bf16 X (m x n) and symmetric out_2 (m x m) (triton_muon.py:281-310)."""
     _check_bf16_2d(X, "X")
     _check_bf16_2d(out_2, "out_2")
+    if _ns_direct(_NS_UPDATE, X, out_2, out, a, 0.0, 0.0):
+        return
     m, n = X.shape
     mp, np_ = _rup(m, 128), _rup(n, 128)
     Xp = _padded(X, mp, np_)
@@ -244,6 +328,8 @@ def solve_ns_kernel_3(X: torch.Tensor, out_2: torch.Tensor, a: float, out: torch
 def newton_shultz_step(X: torch.Tensor, a: float, b: float, c: float, out: torch.Tensor) -> None:
     """One Newton-Schulz iteration out = a*X + (b*A + c*A@A) @ X, A = X @ X.T (triton_muon.py:313-325)."""
     _check_bf16_2d(X, "X")
+    if _ns_direct(_NS_STEP, X, None, out, a, b, c):
+        return
     m, n = X.shape
     mp, np_ = _rup(m, 128), _rup(n, 128)
     dev = X.device
