@@ -50,6 +50,8 @@ typedef short i16x4_t __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) i16x4_t* lds_i16x4_ptr_t;
 typedef __attribute__((address_space(3))) void* lds_ptr_t;
 
+constexpr int kStoreThrough = 16;  // cache policy bits of a store: sc1 (agent scope, written through)
+
 // Element offset of (r, c) in a fragment-major matrix of `rows` rows.
 __device__ __forceinline__ int foff(int rows, int r, int c) {
     return (((c >> 4) * (rows >> 5) + (r >> 5)) << 9) + (((c >> 3) & 1) << 8) + ((r & 31) << 3) + (c & 7);
@@ -321,6 +323,7 @@ struct DirectGemm {
     // another (each such read is a memory latency of about 0.6 us).
     int mp, np, tiles;
     uint32_t stride;  // workspace bytes of a matrix / 256
+    int total;        // launch blocks
     float alpha;  // coefficient on the accumulator (polynomial)
     float beta;   // coefficient on A (polynomial) or X (update, apply)
     float keep;   // apply: 1 - lr * weight_decay
@@ -345,7 +348,11 @@ __global__ __launch_bounds__(64, 2) void direct_gemm_kernel(char* ws, const Dire
         if (g.found_inf && *g.found_inf != 0.0f) return;
     }
     const int lane = threadIdx.x;
-    const int block = xcd_contiguous(blockIdx.x, gridDim.x);
+    // All scalar arguments in one read (the compiler would fetch them where
+    // they are first used, each a latency of its own: 1 us of a 50 us step).
+    asm volatile("" ::"s"(g.mp), "s"(g.np), "s"(g.tiles), "s"(g.stride), "s"(g.cur), "s"(g.super), "s"(g.total), "s"(ws),
+                 "s"(g.alpha), "s"(g.beta));
+    const int block = xcd_contiguous(blockIdx.x, g.total);
     int mi, t, ty, tx, mp = g.mp, np = g.np;
     uint32_t region;
     if (g.tiles > 0) {
@@ -539,9 +546,9 @@ __global__ __launch_bounds__(64, 2) void direct_gemm_kernel(char* ws, const Dire
                             const float o = __builtin_fmaf(-d.slr, u[e], pv * g.keep);
                             const int so = (a * 32 + q * 8 + e) * C + c * 32;
                             if (bf)
-                                __builtin_amdgcn_raw_buffer_store_b16(short(f32_to_bf16(o)), rp, at0 * 2, so * 2, 0);
+                                __builtin_amdgcn_raw_buffer_store_b16(short(f32_to_bf16(o)), rp, at0 * 2, so * 2, kStoreThrough);
                             else
-                                __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(o), rp, at0 * 4, so * 4, 0);
+                                __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(o), rp, at0 * 4, so * 4, kStoreThrough);
                             if (d.upd) __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(u[e]), ru, at0 * 4, so * 4, 0);
                         }
                     }
@@ -640,6 +647,12 @@ __global__ __launch_bounds__(64, 2) void direct_gemm_kernel(char* ws, const Dire
     uint16_t* const across = MODE == DM_GRAM ? A : MODE == DM_POLY ? B
                            : reinterpret_cast<uint16_t*>(base + (g.cur ? 0 : direct_off_xt1(mp, np)));
     uint16_t* const along = MODE == DM_GRAM ? A : MODE == DM_POLY ? B : X;
+    // Stores write through the L2 (kStoreThrough): the tiles of a small launch
+    // end together, and what is still dirty in the L2s is written back before
+    // the next launch may begin (2 x 512 x 2048 step 115 -> 109 us, 4 x 768 x
+    // 768 160 -> 152, 2048 x 2048 325 -> 311).
+    const __amdgpu_buffer_rsrc_t r_across = rsrc(across, int64_t(xrows) * (SYM ? mp : yrows) * 2);
+    const __amdgpu_buffer_rsrc_t r_along = rsrc(along, int64_t(yrows) * (SYM ? mp : xrows) * 2);
 #pragma unroll
     for (int a = 0; a < F; ++a)
 #pragma unroll
@@ -651,7 +664,9 @@ __global__ __launch_bounds__(64, 2) void direct_gemm_kernel(char* ws, const Dire
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
                 const uint2 w = value(a, c, q);
-                *reinterpret_cast<uint2*>(across + foff(xrows, x0 + (lane & 31), y0 + q * 8 + (lane >> 5) * 4)) = w;
+                __builtin_amdgcn_raw_buffer_store_b64(u32x2_t{w.x, w.y}, r_across,
+                                                      foff(xrows, x0 + (lane & 31), y0 + q * 8 + (lane >> 5) * 4) * 2, 0,
+                                                      kStoreThrough);
                 *reinterpret_cast<uint2*>(&tr[(lane & 31) * LD + q * 8 + (lane >> 5) * 4]) = w;
             }
             if (!both) continue;
@@ -665,8 +680,8 @@ __global__ __launch_bounds__(64, 2) void direct_gemm_kernel(char* ws, const Dire
                     uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4_ptr_t)(lds_ptr_t)(const_cast<uint16_t*>(s0))));
                 const uint2 hi = __builtin_bit_cast(
                     uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4_ptr_t)(lds_ptr_t)(const_cast<uint16_t*>(s0 + 4 * LD))));
-                *reinterpret_cast<uint4*>(along + foff(yrows, y0 + band * 16 + j, x0 + xc)) =
-                    make_uint4(lo.x, lo.y, hi.x, hi.y);
+                __builtin_amdgcn_raw_buffer_store_b128(u32x4_t{lo.x, lo.y, hi.x, hi.y}, r_along,
+                                                       foff(yrows, y0 + band * 16 + j, x0 + xc) * 2, 0, kStoreThrough);
             }
         }
 }
@@ -711,6 +726,7 @@ hipError_t launch_direct(const DirectBatch& b, char* ws, const DirectGemm& g, do
     // m >= 1024 of 256 (the tiles the staged kernels use there).
     const int square = (MODE == DM_UPDATE || MODE == DM_APPLY) && m >= 1024 ? 256 : 128;
     ga.super = square / T;
+    ga.total = int(total);
     if (b.uniform) {
         ga.mp = b.d[0].mp;
         ga.np = b.d[0].np;
