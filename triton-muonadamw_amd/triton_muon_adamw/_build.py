@@ -26,6 +26,7 @@ INCLUDE = REPO / "include"
 BUILD_DIR = ROOT_PKG / "_build"
 LIB_NAME = "libmuonadamw_amd.so"
 LIB_PATH = PKG_DIR / LIB_NAME
+LAYOUT_PATH = PKG_DIR / "_layout.so"  # CPython module (csrc/layout.cpp), see _lib.layout
 
 ARCH = "gfx950"
 
@@ -129,13 +130,37 @@ def _check_untracked_reads(src: Path, verbose: bool, out_dir: Path = BUILD_DIR) 
                            + "\n".join(rep.hazards[:20]))
 
 
+def _build_layout(verbose: bool) -> None:
+    """The CPython module: host C++ against torch's headers (no HIP)."""
+    import sysconfig
+
+    import torch
+    from torch.utils.cpp_extension import include_paths
+
+    cxx = os.environ.get("CXX") or shutil.which("g++") or shutil.which("c++")
+    if not cxx:
+        raise RuntimeError("no C++ compiler for triton_muon_adamw._layout")
+    lib_dir = Path(torch.__file__).resolve().parent / "lib"
+    tmp = LAYOUT_PATH.with_name(LAYOUT_PATH.name + ".tmp")
+    cmd = [cxx, "-O2", "-std=c++17", "-shared", "-fPIC", "-Wall",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+           *(f"-isystem{d}" for d in include_paths()), f"-I{sysconfig.get_paths()['include']}",
+           str(CSRC / "layout.cpp"), f"-L{lib_dir}", "-lc10", "-ltorch_cpu", "-ltorch_python", "-o", str(tmp)]
+    if verbose:
+        print(" ".join(cmd), flush=True)
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    if res.returncode != 0:
+        raise RuntimeError(f"layout.cpp failed to build:\n{res.stdout}\n{res.stderr}")
+    os.replace(tmp, LAYOUT_PATH)
+
+
 def build(verbose: bool = False) -> Path:
     """Compile every source and link the shared library; returns its path."""
     BUILD_DIR.mkdir(exist_ok=True)
     objs = []
-    jobs = min(len(SOURCES) + 1, max(1, os.cpu_count() or 1))
+    jobs = min(len(SOURCES) + 2, max(1, os.cpu_count() or 1))
     with cf.ThreadPoolExecutor(max_workers=jobs) as ex:
-        futs = []
+        futs = [ex.submit(_build_layout, verbose)]
         for name in SOURCES:
             src = CSRC / name
             obj = BUILD_DIR / (name + ".o")

@@ -203,6 +203,30 @@ def layout_key(p: torch.Tensor) -> tuple:
     return (id(p), p.data_ptr(), p.dtype, p.shape, p.stride(), g.data_ptr(), g.dtype, g.shape, g.stride())
 
 
+_layout = None
+
+
+def layout(params) -> tuple[list, object]:
+    """``(active, key)``: the parameters that have a gradient, and what a launch
+    plan of them assumes (``layout_key`` of each), in a form that compares
+    equal exactly while none of it changed.  Read natively
+    (``csrc/layout.cpp``) from a list of plain tensors and parameters; tensor
+    subclasses and other sequences attribute by attribute."""
+    global _layout
+    if _layout is None:
+        try:
+            from . import _layout as module
+        except ImportError as e:
+            raise RuntimeError("_layout is not built; run __graft_entry__.build() "
+                               "(or python -m triton_muon_adamw._build)") from e
+        _layout = module
+    found = _layout.layout(params)
+    if found is None:
+        active = [p for p in params if p.grad is not None]
+        found = active, tuple(layout_key(p) for p in active)
+    return found
+
+
 def check_not_capturing(branch: str) -> None:
     """Launch plans and device step counters are made by eager steps only: a
     graph replays the pointers, scalars and table upload recorded at capture."""
@@ -216,6 +240,27 @@ def check_not_capturing(branch: str) -> None:
 def stream_handle(device: torch.device) -> int:
     """hipStream_t of torch's current stream on ``device`` (0 = null stream)."""
     return torch.cuda.current_stream(device).cuda_stream
+
+
+def raw_stream(device: torch.device) -> int:
+    """``stream_handle`` of a device with an index, without making a Stream object."""
+    return torch._C._cuda_getCurrentRawStream(device.index)
+
+
+class _NoGuard:
+    def __enter__(self):
+        return None
+
+    def __exit__(self, *exc):
+        return False
+
+
+_no_guard = _NoGuard()
+
+
+def device_guard(device: torch.device):
+    """``torch.cuda.device(device)``, for nothing where that is the current device already."""
+    return _no_guard if torch._C._cuda_getDevice() == device.index else torch.cuda.device(device)
 
 
 _HIP_STREAM_NON_BLOCKING = 1

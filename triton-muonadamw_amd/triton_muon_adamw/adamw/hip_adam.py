@@ -51,17 +51,17 @@ def solve_adamw_step(matrix: torch.Tensor, gradient: torch.Tensor, m: torch.Tens
         if t.numel() != matrix.numel() or t.device != matrix.device:
             raise ValueError(f"{name} must match the parameter's numel and device")
     lib = _lib.load()
-    with torch.cuda.device(matrix.device):
+    with _lib.device_guard(matrix.device):
         st = lib.mamw_adamw_tensor_step(
             matrix.data_ptr(), gradient.data_ptr(), m.data_ptr(), v.data_ptr(), matrix.numel(),
-            lr, bias1, bias2, beta1, beta2, weight_decay, eps, _lib.stream_handle(matrix.device))
+            lr, bias1, bias2, beta1, beta2, weight_decay, eps, _lib.raw_stream(matrix.device))
     _lib.check(st, "mamw_adamw_tensor_step")
 
 
 class _DevicePlan:
     """Packed tensor table of one device, resident in device memory."""
 
-    __slots__ = ("device", "table", "n_tensors", "n_blocks")
+    __slots__ = ("device", "table", "table_ptr", "home", "n_tensors", "n_blocks")
 
     def __init__(self, device: torch.device, entries: list[tuple[torch.Tensor, ...]]):
         lib = _lib.load()
@@ -83,6 +83,8 @@ class _DevicePlan:
                    "mamw_adamw_table_pack_ex")
         self.device = device
         self.table = torch.empty(host.numel(), dtype=torch.uint8, device=device)
+        self.table_ptr = self.table.data_ptr()
+        self.home = _lib.raw_stream(device)  # the stream the table's memory belongs to
         with torch.cuda.device(device):
             self.table.copy_(host, non_blocking=True)
         self.n_tensors = n
@@ -91,11 +93,12 @@ class _DevicePlan:
     def launch_stream(self) -> int:
         """Handle of the current stream, on which the table is about to be
         read.  The table was allocated on the stream current when it was packed;
-        recording this one keeps torch's allocator from reusing the table's
+        recording another one keeps torch's allocator from reusing the table's
         memory, once the plan is replaced, before the launch has run."""
-        s = torch.cuda.current_stream(self.device)
-        self.table.record_stream(s)
-        return s.cuda_stream
+        handle = _lib.raw_stream(self.device)
+        if handle != self.home:
+            self.table.record_stream(torch.cuda.current_stream(self.device))
+        return handle
 
 
 class HipAdamW:
@@ -190,21 +193,16 @@ class HipAdamW:
         else:
             self._dev_steps: dict[torch.device, torch.Tensor] = {}
 
-    def _refresh_plans(self, active: list[nn.Parameter]) -> None:
-        key = tuple(_lib.layout_key(p) for p in active)
-        if key != self._plan_key:
-            _lib.check_not_capturing("AdamW")
-            self._plan_key = None
-            self._build_plans(active)
-            self._plan_key = key
-
     def _plan(self) -> list[nn.Parameter]:
         """The parameters that have a gradient, with their launch plan checked
         (rebuilt when any of them changed): argument errors raise here, before
         anything of the step is queued or counted."""
-        active = [p for p in self.model_params if p.grad is not None]
-        if active:
-            self._refresh_plans(active)
+        active, key = _lib.layout(self.model_params)
+        if active and key != self._plan_key:
+            _lib.check_not_capturing("AdamW")
+            self._plan_key = None
+            self._build_plans(active)
+            self._plan_key = key
         return active
 
     @torch.no_grad()
@@ -237,9 +235,9 @@ class HipAdamW:
             bias1 = 1 - self.beta1**self._step_host
             bias2 = 1 - self.beta2**self._step_host
             for plan in self._plans:
-                with torch.cuda.device(plan.device):
+                with _lib.device_guard(plan.device):
                     st = lib.mamw_adamw_mt_step(
-                        plan.table.data_ptr(), plan.n_tensors, plan.n_blocks, self.lr, bias1, bias2,
+                        plan.table_ptr, plan.n_tensors, plan.n_blocks, self.lr, bias1, bias2,
                         self.beta1, self.beta2, self.weight_decay, self.eps, plan.launch_stream())
                 _lib.check(st, "mamw_adamw_mt_step")
             return

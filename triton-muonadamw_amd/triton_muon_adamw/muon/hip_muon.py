@@ -255,9 +255,9 @@ def _ns_direct(op: int, X: torch.Tensor, S, out: torch.Tensor, a: float, b: floa
     nbytes = ctypes.c_size_t()
     _lib.check(lib.mamw_ns_direct_workspace_bytes(m, n, ctypes.byref(nbytes)), "mamw_ns_direct_workspace_bytes")
     ws = torch.empty(nbytes.value, dtype=torch.uint8, device=dev)
-    with torch.cuda.device(dev):
+    with _lib.device_guard(dev):
         st = lib.mamw_ns_direct(op, X.data_ptr(), S.data_ptr() if S is not None else None, out.data_ptr(), m, n, a, b,
-                                c, ws.data_ptr(), nbytes.value, _lib.stream_handle(dev))
+                                c, ws.data_ptr(), nbytes.value, _lib.raw_stream(dev))
     _lib.check(st, "mamw_ns_direct")
     torch.autograd.graph.increment_version(out)  # written in place, as copy_ records
     return True
@@ -376,8 +376,8 @@ def muon_step(weights: torch.Tensor, grad: torch.Tensor, momentum: torch.Tensor,
     nbytes = _direct_workspace_bytes(arr, 1, steps) if direct else _workspace_bytes(1, R, C, steps)
     ws = torch.empty(nbytes, dtype=torch.uint8, device=weights.device)
     args = (arr, 1, lr, weight_decay, beta, int(bool(nesterov)), a, b, c, steps, eps, ws.data_ptr(), nbytes)
-    with torch.cuda.device(weights.device):
-        s = _lib.stream_handle(weights.device)
+    with _lib.device_guard(weights.device):
+        s = _lib.raw_stream(weights.device)
         st = lib.mamw_muon_direct_step(*args, None, None, s) if direct else lib.mamw_muon_step(*args, s)
     _lib.check(st, "mamw_muon_step")
 
@@ -622,6 +622,7 @@ class HipMuon:
         self._calls: list[_Call] = []
         self._launches: list[_Launch] = []
         self._ws: dict = {}  # device (launches in order) or (device, shape class) (own streams) -> workspace
+        self._ws_home: dict = {}  # same keys -> handle of the stream the workspace's memory belongs to
         self._concurrent = False
         # (device, shape class) -> side stream, or None: the caller's stream (of a staged class)
         self._lanes: dict = {}
@@ -719,11 +720,14 @@ class HipMuon:
                 launches.append(_Launch(dev, arr, n, run[0].direct, lane, key))
         for key in [k for k in self._ws if k not in need]:
             del self._ws[key]
+            self._ws_home.pop(key, None)
         for key, nbytes in need.items():
             ws = self._ws.get(key)
             if ws is None or ws.numel() < nbytes:
                 self._ws[key] = None
-                self._ws[key] = torch.empty(nbytes, dtype=torch.uint8, device=key[0] if isinstance(key, tuple) else key)
+                dev = key[0] if isinstance(key, tuple) else key
+                self._ws[key] = torch.empty(nbytes, dtype=torch.uint8, device=dev)
+                self._ws_home[key] = _lib.raw_stream(dev)
         self._calls = calls
         self._launches = launches
         self._concurrent = concurrent
@@ -745,10 +749,10 @@ class HipMuon:
         """The parameters that have a gradient, with the launch plan checked
         (rebuilt when any of them changed): argument errors raise here, before
         anything of the step is queued."""
-        active = [p for p in self.model_params if p.grad is not None]
+        active, layouts = _lib.layout(self.model_params)
         if not active:
             return active
-        key = (self.adjust_lr_fn, self.steps, tuple(_lib.layout_key(p) for p in active))
+        key = (self.adjust_lr_fn, self.steps, layouts)
         if key != self._plan_key:
             _lib.check_not_capturing("Muon")
             self._plan_key = None
@@ -785,7 +789,7 @@ class HipMuon:
                     self.eps, ws.data_ptr(), ws.numel())
             gs, fi = amp_ptrs[call.device] if amp else (None, None)
             scaler = (gs.data_ptr() if gs is not None else None, fi.data_ptr() if fi is not None else None)
-            with torch.cuda.device(call.device):
+            with _lib.device_guard(call.device):
                 if call.direct:
                     st = lib.mamw_muon_direct_step(*args, *scaler, stream_handle)
                 elif not amp:
@@ -796,9 +800,8 @@ class HipMuon:
 
         if not self._concurrent:
             for call in self._launches:
-                ws, cur = self._ws[call.ws_key], torch.cuda.current_stream(call.device)
-                ws.record_stream(cur)  # allocated under the stream current when the plan was built
-                launch(call, ws, cur.cuda_stream)
+                handle = _lib.raw_stream(call.device)
+                launch(call, self._workspace(call.ws_key, call.device, handle), handle)
             return
         # Concurrent shape classes (lanes from _lanes): the largest on the
         # caller's current stream, the others on side streams.  Every side
@@ -817,12 +820,19 @@ class HipMuon:
                         t.record_stream(s)
         for call in self._launches:
             s = call.lane
-            if s is None:
-                s = torch.cuda.current_stream(call.device)
-            self._ws[call.ws_key].record_stream(s)
-            launch(call, self._ws[call.ws_key], s.cuda_stream)
+            handle = _lib.raw_stream(call.device) if s is None else s.cuda_stream
+            launch(call, self._workspace(call.ws_key, call.device, handle, s), handle)
         for (dev, _), s in side.items():
             torch.cuda.current_stream(dev).wait_stream(s)
+
+    def _workspace(self, key, device: torch.device, handle: int, stream=None) -> torch.Tensor:
+        """The workspace ``key`` for a launch on ``stream`` (the current one by
+        default; ``handle`` its handle): recorded there unless its memory
+        belongs to that stream, the one current when the plan was built."""
+        ws = self._ws[key]
+        if handle != self._ws_home[key]:
+            ws.record_stream(torch.cuda.current_stream(device) if stream is None else stream)
+        return ws
 
     def zero_grad(self, set_to_none: bool = False):
         """Resets gradients back to zero (the reference's behaviour), or to None
