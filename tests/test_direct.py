@@ -80,6 +80,38 @@ def test_direct_equals_staged(gpu, shapes, pd, gd, shift, ns_steps, nesterov):
                 assert torch.equal(a[k], b[k]), (i, shapes[i], what)
 
 
+# A last round of few 256-wide tiles as 128-wide ones (muon.hip launch_gemm):
+# every product of one 2048 x 2300 (36 and 72 tiles, no full round); 260
+# symmetric tiles, four after a full round, lower-triangle A and B; 360 (104
+# after a full round) with ragged edges and both orientations.
+@pytest.mark.gpu
+@pytest.mark.parametrize("shapes", [[(2048, 2300)], [(1024, 1280)] * 26, [(2100, 2100)] * 4 + [(2100, 2100)] * 4],
+                         ids=lambda s: f"{len(s)}x{s[0][0]}x{s[0][1]}")
+def test_split_last_round_equals_direct(gpu, shapes):
+    """Bit for bit against the direct path, which has neither tiles nor lower triangles in common with it."""
+    lib = _lib.load()
+    stream = torch.cuda.current_stream(gpu).cuda_stream
+    hyper = (2e-2, 0.1, 0.95, 1, *COEFFS, 3, 1e-7)
+    mine, ref = (_make(shapes, gpu, F32, F32, 0, True) for _ in range(2))
+    n = hip_muon._workspace_bytes(len(shapes), *shapes[0], 3)
+    ws = torch.full((n,), 0xFF, dtype=torch.uint8, device=gpu)
+    _lib.prof_start()
+    _lib.check(lib.mamw_muon_step(_arr(mine), len(shapes), *hyper, ws.data_ptr(), n, stream), "staged")
+    _lib.prof_stop()
+    recs = [r for r in _lib.prof_collect() if r["kernel"].startswith("ns_gemm")]
+    assert len(recs) == 9  # one per product, named after its whole rounds where it has any
+    assert {r["variant"] // 8 for r in recs if r["kernel"] in ("ns_gemm_kernel:gram", "ns_gemm_kernel:poly")} == {
+        128 if len(shapes) == 1 else 256}
+    arr = _arr(ref)
+    n = hip_muon._direct_workspace_bytes(arr, len(shapes), 3)
+    ws = torch.empty(n, dtype=torch.uint8, device=gpu)
+    _lib.check(lib.mamw_muon_direct_step(arr, len(shapes), *hyper, ws.data_ptr(), n, None, None, stream), "direct")
+    torch.cuda.synchronize()
+    for a, b in zip(mine, ref):
+        for k in (0, 2, 3):
+            assert torch.equal(a[k], b[k])
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("inf", [0.0, 1.0])
 def test_direct_gradient_scaler_step(gpu, inf):
@@ -152,7 +184,7 @@ def test_direct_rejects_before_hip():
 def test_direct_choice():
     """Small groups go direct, groups that fill the GPU with staged tiles do not; a set of classes goes as one."""
     pays = hip_muon.direct_pays
-    for shape, count in (((512, 2048), 2), ((3072, 768), 1), ((10, 517), 32), ((2048, 2048), 1), ((1024, 4096), 1)):
+    for shape, count in (((512, 2048), 2), ((3072, 768), 1), ((10, 517), 32), ((1536, 1536), 1), ((1024, 4096), 1)):
         assert pays(*shape, count, 256, 5), (shape, count)
     for shape, count in (((512, 2048), 16), ((768, 3072), 12), ((1024, 2048), 8), ((4096, 4096), 1),
                          ((14336, 4096), 1), ((8192, 8256), 1)):

@@ -66,4 +66,16 @@ hipError_t launch(int32_t kernel_id, int32_t variant, double flops, double bytes
     return hipGetLastError();
 }
 
+// One launch of several that make up one record: the first carries the record's
+// start event, the last its stop event (both NULL when profiling is off).
+template <typename Kernel, typename... Args>
+hipError_t launch_part(hipEvent_t start, hipEvent_t stop, Kernel kernel, dim3 grid, dim3 block, hipStream_t stream,
+                       Args... args) {
+    if (start || stop)
+        hipExtLaunchKernelGGL(kernel, grid, block, 0, stream, start, stop, 0, args...);
+    else
+        hipLaunchKernelGGL(kernel, grid, block, 0, stream, args...);
+    return hipGetLastError();
+}
+
 }  // namespace mamw

@@ -425,6 +425,7 @@ struct GemmArgs {
     int kmajor;           // GRAM, k-blocked: operands are X^T (lda = its rows), read k-major
     int lower;            // GRAM/POLY, k-blocked: write only the lower triangle (the transposed orientation)
     int a_low;            // POLY/UPDATE/APPLY, k-blocked: the symmetric operand (A; B) holds only its lower triangle
+    int split_first;      // 128-wide tiles: >= 0, the launch's blocks are quarters of the 256-wide tiles from this one on
 };
 
 // Launch block -> (matrix, tile row, tile col).
@@ -445,17 +446,21 @@ struct GemmArgs {
 constexpr int kXcds = 8;
 constexpr int kXcdSlots = 32;
 
-template <bool SYM, int kGroupM>
-__device__ __forceinline__ void decode_tile(const GemmArgs& g, int& bat, int& ti, int& tj) {
+// Blocks before the last, incomplete round keep their order; see above.
+__device__ __forceinline__ int logical_block() {
     const int L = blockIdx.x, total = gridDim.x;
     const int full = (total / (kXcds * kXcdSlots)) * (kXcds * kXcdSlots);
     const int xcd = L % kXcds, j = L / kXcds;
     const int rem = total - full, q = rem / kXcds, r = rem % kXcds;  // the last round: XCD x gets q or q+1
-    const int logical = L < full ? ((j / kXcdSlots) * kXcds + xcd) * kXcdSlots + j % kXcdSlots
-                                 : full + xcd * q + min(xcd, r) + (L - full) / kXcds;
+    return L < full ? ((j / kXcdSlots) * kXcds + xcd) * kXcdSlots + j % kXcdSlots
+                    : full + xcd * q + min(xcd, r) + (L - full) / kXcds;
+}
+
+// T, N: tile rows and columns of a matrix.
+template <bool SYM, int kGroupM>
+__device__ __forceinline__ void decode_tile(const GemmArgs& g, int logical, int T, int N, int& bat, int& ti, int& tj) {
     bat = logical / g.tiles_per_matrix;
     int t = logical - bat * g.tiles_per_matrix;
-    const int T = g.tiles_m;
     if (SYM) {
         // Group of rows [first, first+gs): a triangle (column first+c holds
         // rows first..first+c), then full columns of gs rows.
@@ -479,7 +484,7 @@ __device__ __forceinline__ void decode_tile(const GemmArgs& g, int& bat, int& ti
             ti = first + t % gs;
         }
     } else {
-        const int width = kGroupM * g.tiles_n;
+        const int width = kGroupM * N;
         const int group = t / width, first = group * kGroupM;
         const int gsize = min(T - first, kGroupM);
         const int w = t - group * width;
@@ -665,7 +670,19 @@ __global__ __launch_bounds__(kGemmThreads, BM == 128 ? 2 : 1) void ns_gemm_kerne
         if (g.found_inf && *g.found_inf != 0.0f) return;  // uniform per launch: the whole block leaves
     }
     int bat, ti, tj;
-    decode_tile<SYM, BM == 128 ? 8 : 4>(g, bat, ti, tj);
+    bool in_diag = false;  // a quarter of a diagonal 256-wide tile
+    if (BM == 128 && BN == 128 && KB && g.split_first >= 0) {
+        // Quarter of a 256-wide tile, in that tile's order.  A symmetric
+        // product's diagonal tile has three.
+        const int logical = logical_block(), sub = logical & 3;
+        decode_tile<SYM, 4>(g, g.split_first + (logical >> 2), g.tiles_m / 2, g.tiles_n / 2, bat, ti, tj);
+        in_diag = SYM && ti == tj;
+        if (in_diag && sub == 1) return;
+        ti = 2 * ti + (sub & 1);
+        tj = 2 * tj + (sub >> 1);
+    } else {
+        decode_tile<SYM, BM == 128 ? 8 : 4>(g, logical_block(), g.tiles_m, g.tiles_n, bat, ti, tj);
+    }
     // Uniform by construction; pinned to scalar registers so that every
     // buffer resource derived from them is one (a resource the compiler
     // cannot prove uniform turns each load into a loop over the lanes).
@@ -1204,8 +1221,10 @@ __global__ __launch_bounds__(kGemmThreads, BM == 128 ? 2 : 1) void ns_gemm_kerne
         const int base_tr = int((int64_t(ti) * (BM / 64) * rows_t + int64_t(tj) * BN) * 128);
         const int base_dir = int((int64_t(tj) * (BN / 64) * rows_x + int64_t(ti) * BM) * 128);
         // lower: a symmetric product keeps only its lower triangle (the
-        // transposed orientation of the tiles on and above the diagonal).
-        const bool tr_on = has_tr, dir_on = has_dir && !(SYM && g.lower);
+        // transposed orientation of the tiles on and above the diagonal); a
+        // diagonal block of the lower triangle is whole, so the quarter above
+        // the diagonal of a split one is written both ways.
+        const bool tr_on = has_tr, dir_on = has_dir && (!(SYM && g.lower) || in_diag);
         auto tr_read = [&](int it) {
             const int x = (it % XP) * 32 + (tid >> 3), c = (it / XP) * 8 + (tid & 7);
             return *reinterpret_cast<const uint4*>(TT + x * BM + (((c ^ x ^ (x >> 3)) & (NCH - 1)) << 3));
@@ -1428,54 +1447,94 @@ __global__ __launch_bounds__(256) void transpose_bf16_kernel(const uint16_t* __r
 constexpr int kTile128x192 = 192;
 
 template <int MODE>
-hipError_t launch_gemm(int tile, const GemmArgs& g, const MuonBatchDescs& d, int batch, double flops,
-                       hipStream_t s) {
-    // Products with an epilogue coefficient peel the last two k steps and
-    // prefetch into stage buffer 0 during the last one: K is a multiple of 2 kBK.
-    if (g.K < kBK || g.K % kBK != 0 || (MODE != MODE_GRAM && g.K % (2 * kBK) != 0)) return hipErrorInvalidValue;
-    GemmArgs ga = g;
-    ga.tiles_per_matrix = (MODE == MODE_GRAM || MODE == MODE_POLY) ? g.tiles_m * (g.tiles_m + 1) / 2
-                                                                   : g.tiles_m * g.tiles_n;
-    dim3 grid(unsigned(ga.tiles_per_matrix) * unsigned(batch));
-    const int32_t kid = MODE == MODE_GRAM ? K_NS_GRAM : MODE == MODE_POLY ? K_NS_POLY
-                      : MODE == MODE_UPDATE ? K_NS_UPDATE : K_NS_APPLY;
+constexpr int32_t gemm_kernel_id() {
+    return MODE == MODE_GRAM ? K_NS_GRAM : MODE == MODE_POLY ? K_NS_POLY : MODE == MODE_UPDATE ? K_NS_UPDATE : K_NS_APPLY;
+}
+
+// Profiler variant: tile and the KB, KM, LOW template flags.
+template <int MODE>
+int32_t gemm_variant(int tile, const GemmArgs& g) {
     const bool kb = g.xkb != 0;
     const bool km = MODE == MODE_GRAM && kb && g.kmajor;
     const bool low = MODE != MODE_GRAM && kb && g.a_low;
-    // tile and the KB, KM, LOW template flags
-    const int32_t variant = 8 * tile + (low ? 4 : 0) + (km ? 2 : 0) + (kb ? 1 : 0);
-    const dim3 block(kGemmThreads);
+    return 8 * tile + (low ? 4 : 0) + (km ? 2 : 0) + (kb ? 1 : 0);
+}
+
+// run(kernel) with the kernel for `tile` and the arguments' layouts.
+template <int MODE, typename Run>
+hipError_t select_kernel(int tile, const GemmArgs& g, Run run) {
+    const bool kb = g.xkb != 0, low = MODE != MODE_GRAM && kb && g.a_low;
     if constexpr (MODE == MODE_UPDATE || MODE == MODE_APPLY) {
         if (tile == kTile128x192) {
             if (!low) return hipErrorInvalidValue;
-            return launch(kid, variant, flops, 0.0, ns_gemm_kernel<128, MODE, true, false, true, 192>, grid, block,
-                          s, ga, d);
+            return run(ns_gemm_kernel<128, MODE, true, false, true, 192>);
         }
     }
     if (tile == kTile128x192) return hipErrorInvalidValue;
+    const bool wide = tile == 256;
     if constexpr (MODE != MODE_GRAM) {
-        if (low) {
-            if (tile == 256)
-                return launch(kid, variant, flops, 0.0, ns_gemm_kernel<256, MODE, true, false, true>, grid, block, s,
-                              ga, d);
-            return launch(kid, variant, flops, 0.0, ns_gemm_kernel<128, MODE, true, false, true>, grid, block, s, ga,
-                          d);
-        }
+        if (low)
+            return wide ? run(ns_gemm_kernel<256, MODE, true, false, true>)
+                        : run(ns_gemm_kernel<128, MODE, true, false, true>);
     }
     if constexpr (MODE == MODE_GRAM) {
-        if (kb && g.kmajor) {
-            if (tile == 256)
-                return launch(kid, variant, flops, 0.0, ns_gemm_kernel<256, MODE, true, true>, grid, block, s, ga, d);
-            return launch(kid, variant, flops, 0.0, ns_gemm_kernel<128, MODE, true, true>, grid, block, s, ga, d);
-        }
+        if (kb && g.kmajor)
+            return wide ? run(ns_gemm_kernel<256, MODE, true, true>) : run(ns_gemm_kernel<128, MODE, true, true>);
     }
-    if (kb) {
-        if (tile == 256)
-            return launch(kid, variant, flops, 0.0, ns_gemm_kernel<256, MODE, true>, grid, block, s, ga, d);
-        return launch(kid, variant, flops, 0.0, ns_gemm_kernel<128, MODE, true>, grid, block, s, ga, d);
+    if (kb) return wide ? run(ns_gemm_kernel<256, MODE, true>) : run(ns_gemm_kernel<128, MODE, true>);
+    return wide ? run(ns_gemm_kernel<256, MODE, false>) : run(ns_gemm_kernel<128, MODE, false>);
+}
+
+template <int MODE>
+hipError_t launch_gemm(int tile, const GemmArgs& g, const MuonBatchDescs& d, int batch, double flops, hipStream_t s) {
+    // Products with an epilogue coefficient peel the last two k steps and
+    // prefetch into stage buffer 0 during the last one: K is a multiple of 2 kBK.
+    if (g.K < kBK || g.K % kBK != 0 || (MODE != MODE_GRAM && g.K % (2 * kBK) != 0)) return hipErrorInvalidValue;
+    constexpr bool SYM = MODE == MODE_GRAM || MODE == MODE_POLY;
+    GemmArgs ga = g;
+    ga.split_first = -1;
+    ga.tiles_per_matrix = SYM ? g.tiles_m * (g.tiles_m + 1) / 2 : g.tiles_m * g.tiles_n;
+    const int total = ga.tiles_per_matrix * batch;
+    constexpr int32_t kid = gemm_kernel_id<MODE>();
+    const dim3 block(kGemmThreads);
+    // A last round of few 256-wide tiles leaves most CUs idle for as long as a
+    // full one (1.33 us a k step).  Its tiles go out as four 128-wide ones each
+    // in a launch of their own: up to 64 tiles have a CU per quarter (0.50 us a
+    // step), up to 128 share one with another (0.88), which pays after a full
+    // round of a symmetric product and, from m = 2048, in a launch of less than
+    // a round (below that m the 256 tile is taken only by groups that measured
+    // faster with it; an update's last 65 to 128 tiles after full rounds stay).
+    // The storage stays that of the 256-wide tiles, and each element its sum.
+    // Steps, whole rounds -> split: 2048 x 2048 632 -> 355 us, 4096 x 2048 799
+    // -> 557, two 4096 x 4096 (272 symmetric tiles) 2850 -> 2607, 26 of 1024 x
+    // 4096 2805 -> 2704.
+    constexpr int kRound = kXcds * kXcdSlots;
+    const int full = total / kRound * kRound, tail = total - full;
+    const bool large = g.tiles_m >= 8;
+    const bool shared = tail <= 128 && (full > 0 ? SYM : large);
+    if (tile == 256 && g.xkb && tail > 0 && (tail <= 64 || shared)) {
+        GemmArgs gt = ga;
+        gt.split_first = full;
+        gt.tiles_m *= 2;
+        gt.tiles_n *= 2;
+        const dim3 rest{unsigned(4 * tail)};
+        if (full == 0)
+            return select_kernel<MODE>(128, gt, [&](auto kernel) {
+                return launch(kid, gemm_variant<MODE>(128, gt), flops, 0.0, kernel, rest, block, s, gt, d);
+            });
+        hipEvent_t e0 = nullptr, e1 = nullptr;  // one record for both
+        const bool rec = prof_take(&e0, &e1);
+        hipError_t e = select_kernel<MODE>(256, ga, [&](auto kernel) {
+            return launch_part(e0, nullptr, kernel, dim3{unsigned(full)}, block, s, ga, d);
+        });
+        if (e != hipSuccess) return e;
+        e = select_kernel<MODE>(128, gt, [&](auto kernel) { return launch_part(nullptr, e1, kernel, rest, block, s, gt, d); });
+        if (e == hipSuccess && rec) prof_push(kid, gemm_variant<MODE>(256, ga), flops, 0.0, e0, e1);
+        return e;
     }
-    if (tile == 256) return launch(kid, variant, flops, 0.0, ns_gemm_kernel<256, MODE, false>, grid, block, s, ga, d);
-    return launch(kid, variant, flops, 0.0, ns_gemm_kernel<128, MODE, false>, grid, block, s, ga, d);
+    return select_kernel<MODE>(tile, ga, [&](auto kernel) {
+        return launch(kid, gemm_variant<MODE>(tile, ga), flops, 0.0, kernel, dim3{unsigned(total)}, block, s, ga, d);
+    });
 }
 
 GemmArgs gram_args(const uint16_t* X, uint16_t* A, int64_t mp, int64_t kp, int tile) {

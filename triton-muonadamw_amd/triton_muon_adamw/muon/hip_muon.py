@@ -87,12 +87,21 @@ def _direct_workspace_bytes(arr, count: int, ns_steps: int) -> int:
 # 101, two 198 / 116, eight 238 / 228, sixteen 328 / 374; 768 x 3072 one 268 /
 # 151, eight 438 / 518; 2048 x 2048 one 632 / 331, four 795 / 1088.
 
-def _staged_product_us(tile: int, tiles: int, k: int, cus: int) -> float:
+def _staged_product_us(tile: int, tiles: int, k: int, cus: int, sym: bool = False, large: bool = False) -> float:
     """One staged product: whole rounds of its grid (one 256-wide or two
     128-wide workgroups per CU; a 128-wide workgroup alone on its CU is
-    faster), a k step of 64 at 1.33, 0.88 or 0.50 us, and 3.5 us a launch."""
+    faster), a k step of 64 at 1.33, 0.88 or 0.50 us, and 3.5 us a launch.
+    ``sym``, ``large`` (m >= 2048): what decides whether a last round of few
+    256-wide tiles runs as 128-wide ones (launch_gemm)."""
     if tile == 256:
-        rounds = -(-tiles // cus) * 1.33
+        full, rest = divmod(tiles, cus)
+        if 0 < rest <= 64:
+            last = 0.50
+        elif 0 < rest <= 128 and (sym if full else large):
+            last = 0.88
+        else:
+            last = 1.33 if rest else 0.0
+        rounds = full * 1.33 + last
     else:
         full, rest = divmod(tiles, 2 * cus)
         rounds = full * 0.88 + (0.0 if rest == 0 else 0.50 if rest <= cus else 0.88)
@@ -114,8 +123,9 @@ def _staged_us(m: int, n: int, count: int, cus: int) -> float:
     utile = 256 if (tile == 128 and m >= 1024 and mp % 256 == 0 and np_ % 256 == 0) else tile
     tm = mp // tile
     sym = count * tm * (tm + 1) // 2
-    return (5 * (_staged_product_us(tile, sym, np_, cus) + _staged_product_us(tile, sym, mp, cus)
-                 + _staged_product_us(utile, count * (mp // utile) * (np_ // utile), mp, cus))
+    large = mp >= 2048
+    return (5 * (_staged_product_us(tile, sym, np_, cus, True, large) + _staged_product_us(tile, sym, mp, cus, True, large)
+                 + _staged_product_us(utile, count * (mp // utile) * (np_ // utile), mp, cus, False, large))
             + 8e-6 * count * mp * np_ + 12)
 
 
