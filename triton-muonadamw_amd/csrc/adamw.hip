@@ -80,8 +80,11 @@ __device__ __forceinline__ void adamw_elem(float& p, float g, float& m, float& v
 
 // Streaming 16-byte accesses: every byte is touched once, so the loads and
 // stores are non-temporal (measured: +6-8 points of HBM bandwidth over plain
-// accesses on this kernel; either half alone gains nothing).
-typedef float nt_f4 __attribute__((ext_vector_type(4)));
+// accesses on this kernel; either half alone gains nothing).  The types ask for
+// the element's alignment only: gfx950 takes the wide access at any address,
+// and the instructions are those of the aligned types.
+typedef float nt_f4 __attribute__((ext_vector_type(4), aligned(4)));
+typedef unsigned int nt_u2 __attribute__((ext_vector_type(2), aligned(2)));
 __device__ __forceinline__ float4 nt_load(const float4* q) {
     const nt_f4 v = __builtin_nontemporal_load(reinterpret_cast<const nt_f4*>(q));
     return make_float4(v.x, v.y, v.z, v.w);
@@ -104,7 +107,6 @@ __device__ __forceinline__ void adamw_vec(float4& p, float4 g, float4& m, float4
 template <bool BF16>
 __device__ __forceinline__ float4 ld4(const void* base, int64_t i) {
     if constexpr (BF16) {
-        typedef unsigned int nt_u2 __attribute__((ext_vector_type(2)));
         const nt_u2 w = __builtin_nontemporal_load(reinterpret_cast<const nt_u2*>(base) + i);
         return make_float4(bf16_to_f32(w.x & 0xffffu), bf16_to_f32(w.x >> 16), bf16_to_f32(w.y & 0xffffu),
                            bf16_to_f32(w.y >> 16));
@@ -115,7 +117,6 @@ __device__ __forceinline__ float4 ld4(const void* base, int64_t i) {
 template <bool BF16>
 __device__ __forceinline__ void st4(void* base, int64_t i, float4 x) {
     if constexpr (BF16) {
-        typedef unsigned int nt_u2 __attribute__((ext_vector_type(2)));
         const nt_u2 w = {pack_bf16x2(x.x, x.y), pack_bf16x2(x.z, x.w)};
         __builtin_nontemporal_store(w, reinterpret_cast<nt_u2*>(base) + i);
     } else {
@@ -140,6 +141,12 @@ __device__ __forceinline__ void st1(void* base, int64_t i, float x) {
 // Update elements [start, start + len) of tensor r (len <= kAdamWChunk); PB /
 // GB: the parameter / gradient hold bf16.  The arithmetic is the fp32 one in
 // every case.
+//
+// Buffers that do not lie on 4-element boundaries: with a bf16 one among them
+// the accesses are wide all the same (256 tensors of 1e3 to 4e6 elements packed
+// end to end, bf16 parameters and gradients: single elements 528 us, wide
+// 494); with fp32 alone single elements move whole 256-byte runs per wavefront
+// and lose nothing (662 us, wide 661).
 template <bool PB, bool GB>
 __device__ __forceinline__ void adamw_chunk(const AdamWRec& r, int64_t start, int len,
                                             const AdamWConsts& c) {
@@ -150,7 +157,8 @@ __device__ __forceinline__ void adamw_chunk(const AdamWRec& r, int64_t start, in
     float4* V4 = reinterpret_cast<float4*>(V);
     // Vector index i covers elements start + 4i .. +3 (start is a multiple of 4).
     const int64_t q0 = start >> 2;
-    if (r.vec_ok && len == kAdamWChunk) {
+    const bool wide = PB || GB || r.vec_ok;
+    if (wide && len == kAdamWChunk) {
         float4 p[kAdamWUnroll], g[kAdamWUnroll], m[kAdamWUnroll], v[kAdamWUnroll];
 #pragma unroll
         for (int u = 0; u < kAdamWUnroll; ++u) {
@@ -171,7 +179,7 @@ __device__ __forceinline__ void adamw_chunk(const AdamWRec& r, int64_t start, in
         return;
     }
     int scalar_from = 0;
-    if (r.vec_ok) {
+    if (wide) {
         const int nv = len >> 2;
         for (int i = tid; i < nv; i += kAdamWThreads) {
             float4 p = ld4<PB>(r.p, q0 + i), m = nt_load(M4 + i), v = nt_load(V4 + i);
