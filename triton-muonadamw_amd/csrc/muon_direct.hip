@@ -340,7 +340,7 @@ template <int MODE, int T, bool ROWMAJOR = false>
 __global__ __launch_bounds__(64, 2) void direct_gemm_kernel(char* ws, const DirectGemm g, const DirectIndex ix) {
     constexpr bool SYM = MODE == DM_GRAM || MODE == DM_POLY;
     constexpr int F = T / 32;              // fragments per tile edge
-        constexpr int D = T == 32 ? 4 : 2;     // panels of 64 k in the register ring
+    constexpr int D = T == 32 ? 4 : 2;     // panels of 64 k in the register ring
     // Halves per LDS row of a 32 x 32 fragment; rows read as 16-byte chunks are aligned.
     constexpr int LD = ROWMAJOR ? 40 : 36;
     __shared__ __attribute__((aligned(16))) uint16_t tr[32 * LD];
