@@ -11,7 +11,9 @@ prep (momentum, Nesterov, bf16, transpose, sum of squares), norm, scale
 (``X / ||X||`` in bf16 and its transpose), then per Newton-Schulz iteration a
 Gram, a polynomial and an update GEMM, the last of which writes the
 parameters.  The reference runs about 30 launches per matrix; here a group of
-up to 32 matrices costs ``3 + 3*ns_steps`` launches.
+up to 32 matrices costs ``3 + 3*ns_steps`` launches.  Few small matrices, of
+any shapes, go out together on the direct path instead (``direct_pays``,
+``direct_set_pays``): ``2 + 3*ns_steps`` launches for up to 64 of them.
 Small steps (``HipMuon.concurrent_flops_limit``) run the shape groups
 concurrently on side streams forked from and joined back into the caller's
 current stream; the results are the same bits as in order.
