@@ -197,6 +197,24 @@ def test_direct_choice():
     assert not both(((1024, 2048, 1), (2048, 4096, 1), (4096, 4096, 1), (1024, 4096, 1)), 256, 5)
 
 
+def test_ns_direct_choice():
+    """Standalone products against the row-major staged kernels, which never
+    split a last round of few 256-wide tiles (GPU times of both paths in
+    ``ns_direct_pays``): one round of 36 to 55 symmetric tiles, of 64 update
+    tiles, and rows that padding takes to 2048."""
+    GRAM, POLY, UPDATE, STEP = range(4)
+    pays = hip_muon.ns_direct_pays
+    for op, m, n in ((GRAM, 1024, 4096), (GRAM, 2048, 8192), (GRAM, 2177, 4096), (GRAM, 2304, 4096),
+                     (GRAM, 2560, 4096), (GRAM, 2560, 8192), (GRAM, 2000, 8192), (POLY, 1024, 1024),
+                     (POLY, 2304, 2304), (POLY, 2560, 2560), (POLY, 3072, 3072), (UPDATE, 768, 3001),
+                     (UPDATE, 2048, 2048), (STEP, 512, 512), (STEP, 2048, 4000), (STEP, 2304, 4096),
+                     (STEP, 2560, 2560)):
+        assert pays(op, m, n, 256), (op, m, n)
+    for op, m, n in ((GRAM, 4096, 4096), (POLY, 4096, 4096), (UPDATE, 2048, 8192), (STEP, 4096, 4096),
+                     (GRAM, 8256, 8256)):
+        assert not pays(op, m, n, 256), (op, m, n)
+
+
 def test_merged_launches():
     """Groups go out together up to the table's size and only where no matrix
     writes what another reads or writes."""

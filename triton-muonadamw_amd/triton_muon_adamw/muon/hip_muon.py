@@ -89,17 +89,19 @@ def _direct_workspace_bytes(arr, count: int, ns_steps: int) -> int:
 # 101, two 198 / 116, eight 238 / 228, sixteen 328 / 374; 768 x 3072 one 268 /
 # 151, eight 438 / 518; 2048 x 2048 one 632 / 331, four 795 / 1088.
 
-def _staged_product_us(tile: int, tiles: int, k: int, cus: int, sym: bool = False, large: bool = False) -> float:
+def _staged_product_us(tile: int, tiles: int, k: int, cus: int, split: bool, sym: bool = False,
+                       large: bool = False) -> float:
     """One staged product: whole rounds of its grid (one 256-wide or two
     128-wide workgroups per CU; a 128-wide workgroup alone on its CU is
     faster), a k step of 64 at 1.33, 0.88 or 0.50 us, and 3.5 us a launch.
-    ``sym``, ``large`` (m >= 2048): what decides whether a last round of few
-    256-wide tiles runs as 128-wide ones (launch_gemm)."""
+    ``split``: k-blocked operands (a step's; those of the standalone products
+    are row-major), whose last round of few 256-wide tiles runs as 128-wide
+    ones; how few, by ``sym`` and ``large`` (m >= 2048) (launch_gemm)."""
     if tile == 256:
         full, rest = divmod(tiles, cus)
-        if 0 < rest <= 64:
+        if split and 0 < rest <= 64:
             last = 0.50
-        elif 0 < rest <= 128 and (sym if full else large):
+        elif split and 0 < rest <= 128 and (sym if full else large):
             last = 0.88
         else:
             last = 1.33 if rest else 0.0
@@ -126,8 +128,9 @@ def _staged_us(m: int, n: int, count: int, cus: int) -> float:
     tm = mp // tile
     sym = count * tm * (tm + 1) // 2
     large = mp >= 2048
-    return (5 * (_staged_product_us(tile, sym, np_, cus, True, large) + _staged_product_us(tile, sym, mp, cus, True, large)
-                 + _staged_product_us(utile, count * (mp // utile) * (np_ // utile), mp, cus, False, large))
+    return (5 * (_staged_product_us(tile, sym, np_, cus, True, True, large)
+                 + _staged_product_us(tile, sym, mp, cus, True, True, large)
+                 + _staged_product_us(utile, count * (mp // utile) * (np_ // utile), mp, cus, True, False, large))
             + 8e-6 * count * mp * np_ + 12)
 
 
@@ -210,17 +213,19 @@ _NS_GRAM, _NS_POLY, _NS_UPDATE, _NS_STEP = range(4)  # MAMW_NS_*
 @functools.lru_cache(maxsize=4096)
 def ns_direct_pays(op: int, m: int, n: int, cus: int) -> bool:
     """Whether a standalone product takes the direct path: the estimates of its
-    products (those of the steps above), and what each path does around them:
-    packing (5 us) there; the copy into ``out``, for the update and the
-    iteration a transpose, and padding here.  Measured staged / direct, us:
-    Gram of 1024 x 4096 44 / 23, 1531 x 3001 50 / 30, 4096 x 4096 91 / 124;
-    polynomial of 1024 15 / 11, 3072 73 / 56, 4096 94 / 121; update of 768 x
-    3001 48 / 22, 2048 x 8192 90 / 105; iteration of 512 x 512 36 / 14, 1024 x
-    4096 86 / 42, 4096 x 4096 295 / 388."""
+    products (those of the steps above; here a last round is never split), and
+    what each path does around them: packing (5 us) there; the copy into
+    ``out``, for the update and the iteration a transpose, and padding here.
+    Measured staged / direct, us: Gram of 1024 x 4096 41 / 23, 1531 x 3001 52 /
+    31, 2304 x 4096 80 / 47, 2560 x 8192 140 / 99, 4096 x 4096 89 / 123;
+    polynomial of 1024 17 / 12, 2304 58 / 33, 2560 67 / 38, 3072 73 / 56, 4096
+    92 / 123; update of 768 x 3001 39 / 21, 2048 x 2048 59 / 34, 2048 x 8192 89 /
+    103; iteration of 512 x 512 35 / 17, 1024 x 4096 82 / 41, 2304 x 4096 203 /
+    131, 4096 x 4096 292 / 393."""
     if max(_rup(m, 64) * _rup(n, 64), _rup(m, 64) ** 2) > 1 << 26:
         return False
     mp, np_ = _rup(m, 128), _rup(n, 128)
-    tile = 256 if m >= 2048 and mp % 256 == 0 else 128
+    tile = 256 if mp >= 2048 and mp % 256 == 0 else 128  # the products see padded matrices
     utile = tile if np_ % 256 == 0 else 128
     sym = (mp // tile) * (mp // tile + 1) // 2
     d, e = _rup(m, 64), _rup(n, 64)
@@ -228,11 +233,11 @@ def ns_direct_pays(op: int, m: int, n: int, cus: int) -> bool:
     s64, s32 = r * (r + 1) // 2, r2 * (r2 + 1) // 2
     u64, u32 = r * (e // 64), r2 * (e // 32)
     products = {
-        _NS_GRAM: (_staged_product_us(tile, sym, np_, cus),
+        _NS_GRAM: (_staged_product_us(tile, sym, np_, cus, False),
                    _direct_product_us(s64, s32, e, s64 * 256.0 * e, s32 * 128.0 * e)),
-        _NS_POLY: (_staged_product_us(tile, sym, mp, cus),
+        _NS_POLY: (_staged_product_us(tile, sym, mp, cus, False),
                    _direct_product_us(s64, s32, d, s64 * 256.0 * d, s32 * 128.0 * d)),
-        _NS_UPDATE: (_staged_product_us(utile, (mp // utile) * (np_ // utile), mp, cus),
+        _NS_UPDATE: (_staged_product_us(utile, (mp // utile) * (np_ // utile), mp, cus, False),
                      _direct_product_us(u64, u32, d, u64 * 256.0 * d, u32 * 128.0 * d)),
     }
     staged = direct = 5.0
