@@ -8,6 +8,7 @@ under either path (one chain of 32x32x16 MFMAs, k ascending), and the epilogues
 round at the same places."""
 
 import ctypes
+import types
 
 import pytest
 import torch
@@ -239,6 +240,54 @@ def test_merged_launches():
     assert runs([a, b]) == [[0], [1]]
     b.arr[0].param += 4
     assert runs([a, b]) == [[0, 1]]
+
+
+@pytest.fixture
+def planner(monkeypatch):
+    """plan(shapes, limit=None, **attributes) -> the HipMuon with its launches
+    planned, on the CPU: 256 CUs, the library's own sizes and choices."""
+    props = types.SimpleNamespace(multi_processor_count=256, total_memory=288 << 30)
+    streams = []
+    monkeypatch.setattr(torch.cuda, "get_device_properties", lambda dev: props)
+    monkeypatch.setattr(_lib, "require_gpu_tensor", lambda t, name: None)
+    monkeypatch.setattr(_lib, "raw_stream", lambda dev: 0)
+    monkeypatch.setattr(_lib, "side_streams", lambda dev, n: [streams.append(n) or f"side{i}" for i in range(n)])
+
+    def plan(shapes, limit=None, **attributes):
+        params = [torch.nn.Parameter(torch.zeros(s)) for s in shapes]
+        for p in params:
+            p.grad = torch.zeros_like(p)
+        opt = hip_muon.HipMuon(params)
+        opt.workspace_limit_bytes = limit
+        for k, v in attributes.items():
+            setattr(opt, k, v)
+        opt._build_calls(params)
+        return opt
+
+    plan.streams = streams
+    return plan
+
+
+@pytest.mark.parametrize("limit_mib", [None, 60, 20, 6, 1])
+@pytest.mark.parametrize("in_order", [False, True])
+def test_launches_keep_to_the_workspace_limit(planner, limit_mib, in_order):
+    """Merged or not, direct or staged: no launch's workspace is over the limit
+    unless one matrix alone needs it on the staged path, and every matrix goes
+    out once, with room for it."""
+    shapes = [(256, 1024)] * 32 + [(256, 768)] * 2 + [(128, 8192), (8192, 128)]
+    limit = None if limit_mib is None else limit_mib << 20
+    opt = planner(shapes, limit, **({"concurrent_flops_limit": 0.0} if in_order else {}))
+    assert sum(x.n for x in opt._launches) == len(shapes)
+    assert len({e.param for x in opt._launches for e in x.arr}) == len(shapes)
+    for x in opt._launches:
+        one = {hip_muon._workspace_bytes(1, e.rows, e.cols, 5) for e in x.arr}
+        need = (hip_muon._direct_workspace_bytes(x.arr, x.n, 5) if x.direct
+                else hip_muon._workspace_bytes(x.n, x.arr[0].rows, x.arr[0].cols, 5))
+        assert opt._ws[x.ws_key].numel() >= need
+        if limit is not None:
+            assert need <= limit or not x.direct and x.n == 1 and one == {need}
+    if not in_order and limit is None:  # 36 matrices, one launch
+        assert [(x.n, x.direct, x.lane) for x in opt._launches] == [(36, True, None)]
 
 
 # ---- Standalone products ----------------------------------------------------

@@ -165,11 +165,11 @@ def direct_pays(rows: int, cols: int, count: int, cus: int, ns_steps: int) -> bo
 
 
 @functools.lru_cache(maxsize=1024)
-def direct_set_pays(groups: tuple, cus: int, ns_steps: int) -> bool:
+def direct_set_pays(groups: tuple, cus: int, ns_steps: int, launches: int = 0) -> bool:
     """Whether shape classes that may run beside each other (``groups``: a
-    tuple of (m, n, count)) go out as direct launches of all of them, at most
-    MUON_DIRECT_MAX matrices each, instead of staged groups on their own
-    streams: all or none, since a staged class fills the GPU and a direct one
+    tuple of (m, n, count)) go out as direct launches of all of them
+    (``launches`` of them; 0: as many as MUON_DIRECT_MAX matrices each make),
+    instead of staged groups on their own streams: all or none, since a staged class fills the GPU and a direct one
     beside it costs more than its staged form would (1024-2048-4096-4096-1024
     MLP: 1748 us all staged, 2031 with its three smaller classes direct).
     Staged classes on streams take about 1.15 times their longest class, 0.6
@@ -177,7 +177,7 @@ def direct_set_pays(groups: tuple, cus: int, ns_steps: int) -> bool:
     if not all(_direct_fits(m, n, ns_steps) for m, n, _ in groups):
         return False
     staged = [_staged_us(m, n, count, cus) for m, n, count in groups]
-    launches = -(-sum(count for _, _, count in groups) // _lib.MUON_DIRECT_MAX)
+    launches = max(launches, -(-sum(count for _, _, count in groups) // _lib.MUON_DIRECT_MAX))
     direct = _direct_us(groups) + (launches - 1) * 60
     return direct < 0.9 * max(1.15 * max(staged), 0.6 * sum(staged), 95.0 * len(groups))
 
@@ -572,14 +572,25 @@ def _disjoint(calls) -> bool:
     return True
 
 
-def _merge(calls) -> list[list]:
+def _entries(calls):
+    """The matrices of ``calls`` as one array."""
+    return (_lib.MuonMatrix * sum(c.n for c in calls))(*[e for c in calls for e in c.arr])
+
+
+def _merge(calls, ns_steps: int = 1, limit: int | None = None) -> list[list]:
     """Direct-path ``calls`` as the runs that go out as one launch each: in
-    order, at most MUON_DIRECT_MAX matrices, no memory in common.  (A class's
-    later groups may hold a parameter of an earlier one again.)"""
+    order, at most MUON_DIRECT_MAX matrices and ``limit`` bytes of workspace,
+    no memory in common.  (A class's later groups may hold a parameter of an
+    earlier one again.)"""
+    def fits(run):
+        n = sum(c.n for c in run)
+        return (n <= _lib.MUON_DIRECT_MAX and _disjoint(run)
+                and (limit is None or _direct_workspace_bytes(_entries(run), n, ns_steps) <= limit))
+
     runs: list[list] = []
     for c in calls:
         last = runs[-1] if runs else None
-        if last is not None and sum(x.n for x in last) + c.n <= _lib.MUON_DIRECT_MAX and _disjoint(last + [c]):
+        if last is not None and fits(last + [c]):
             last.append(c)
         else:
             runs.append([c])
@@ -589,11 +600,13 @@ def _merge(calls) -> list[list]:
 class HipMuon:
     """Muon over a list of 2-D parameters, batched by shape on gfx950."""
 
-    # Workspace per launch group is capped at this many bytes (None: 1/20 of
-    # the device's memory, at most 16 GiB; on a 288 GB MI355X 14.4 GB, which
+    # Workspace per launch is capped at this many bytes, except that one matrix
+    # takes what the staged path needs for it (None: 1/20 of the device's
+    # memory, at most 16 GiB; on a 288 GB MI355X 14.4 GB, which
     # lets the 4096 x 14336 Llama-8B matrices run in groups of 32 whose
     # symmetric grids fill whole rounds of the 256 CUs: 3 ms per step faster
-    # than groups of 20).  Within the cap, group_sizes() picks the split.
+    # than groups of 20).  Within the cap, group_sizes() picks the split; a
+    # group whose direct workspace is over it stays staged.
     workspace_limit_bytes: int | None = None
     # A step whose Newton-Schulz work (sum of ns_steps*(3 m^2 n + m^3)) is at
     # most this many flops runs its shape classes concurrently (lanes from
@@ -655,6 +668,11 @@ class HipMuon:
             buf = self.momentum[param] = torch.zeros_like(param, device=param.device, dtype=torch.float32)
         return buf
 
+    def _workspace_limit(self, device: torch.device) -> int:
+        if self.workspace_limit_bytes is not None:
+            return self.workspace_limit_bytes
+        return min(16 << 30, torch.cuda.get_device_properties(device).total_memory // 20)
+
     def _build_calls(self, active: list[nn.Parameter]) -> None:
         groups: dict[tuple, list[nn.Parameter]] = {}
         for p in active:
@@ -674,12 +692,10 @@ class HipMuon:
         calls = []
         flops = sum(self.steps * (3.0 * m * m * n + float(m) ** 3) * len(pl) for (_, m, n), pl in groups.items())
         concurrent = len(groups) > 1 and flops <= self.concurrent_flops_limit
+        limits = {dev: self._workspace_limit(dev) for dev, _, _ in groups}
         for gi, ((dev, m, n), plist) in enumerate(groups.items()):
             one = _workspace_bytes(1, m, n, self.steps)
-            limit = self.workspace_limit_bytes
-            if limit is None:
-                limit = min(16 << 30, torch.cuda.get_device_properties(dev).total_memory // 20)
-            cap = max(1, min(_lib.MUON_MAX_BATCH, limit // max(one, 1)))
+            cap = max(1, min(_lib.MUON_MAX_BATCH, limits[dev] // max(one, 1)))
             cus = torch.cuda.get_device_properties(dev).multi_processor_count
             sizes = iter(group_sizes(len(plist), cap, m, n, cus))
             per = next(sizes)
@@ -706,9 +722,13 @@ class HipMuon:
         for dev in dict.fromkeys(c.device for c in calls):
             cus = torch.cuda.get_device_properties(dev).multi_processor_count
             mine = [c for c in calls if c.device == dev]
-            together = concurrent and direct_set_pays(tuple((c.m, c.n_, c.n) for c in mine), cus, self.steps)
+            fits = {c: _direct_fits(c.m, c.n_, self.steps)
+                    and _direct_workspace_bytes(c.arr, c.n, self.steps) <= limits[dev] for c in mine}
+            together = (concurrent and all(fits.values())
+                        and direct_set_pays(tuple((c.m, c.n_, c.n) for c in mine), cus, self.steps,
+                                            len(_merge(mine, self.steps, limits[dev]))))
             for c in mine:
-                c.direct = together if concurrent else direct_pays(c.m, c.n_, c.n, cus, self.steps)
+                c.direct = together if concurrent else fits[c] and direct_pays(c.m, c.n_, c.n, cus, self.steps)
                 c.ws_bytes = (_direct_workspace_bytes(c.arr, c.n, self.steps) if c.direct
                               else _workspace_bytes(c.n, c.m, c.n_, self.steps))
         self._lanes = {}
@@ -721,17 +741,17 @@ class HipMuon:
         launches, need = [], {}
         for dev in dict.fromkeys(c.device for c in calls):
             mine = [c for c in calls if c.device == dev]
-            for run in (_merge(mine) if concurrent and mine[0].direct else [[c] for c in mine]):
+            merged = concurrent and mine[0].direct
+            for run in (_merge(mine, self.steps, limits[dev]) if merged else [[c] for c in mine]):
                 arr, n, wsb, lane, key = run[0].arr, run[0].n, run[0].ws_bytes, None, dev
                 if concurrent and not run[0].direct:
                     lane, key = self._lanes[(dev, run[0].group)], (dev, run[0].group)
                 if len(run) > 1:
-                    n = sum(c.n for c in run)
-                    arr = (_lib.MuonMatrix * n)(*[e for c in run for e in c.arr])
-                    at = 0
+                    arr, at = _entries(run), 0
                     for c in run:  # the groups' entries are those of the launch
                         c.arr = (_lib.MuonMatrix * c.n).from_buffer(arr, at * ctypes.sizeof(_lib.MuonMatrix))
                         at += c.n
+                    n = at
                     wsb = _direct_workspace_bytes(arr, n, self.steps)
                 need[key] = max(need.get(key, 0), wsb)
                 launches.append(_Launch(dev, arr, n, run[0].direct, lane, key))
