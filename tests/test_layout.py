@@ -80,3 +80,21 @@ def test_layout_of_other_sequences_and_subclasses():
     sub.grad = torch.zeros(3)
     assert _lib.layout([*ps, sub]) == ([*ps[:4], sub], (*ref, _lib.layout_key(sub)))
     assert _lib.layout([]) [0] == []
+
+
+def test_layout_of_a_subclass_gradient():
+    """A gradient of a subclass is read through its own attributes, also on a plain parameter."""
+    class Moved(torch.Tensor):
+        offset = 0
+
+        def data_ptr(self):
+            return super().data_ptr() + self.offset
+
+    ps = _params()
+    ps[1].grad = torch.zeros(3).as_subclass(Moved)
+    active, key = _lib.layout(ps)
+    assert active == ps[:4] and key == tuple(_lib.layout_key(p) for p in ps[:4])
+    ps[1].grad.offset = 4
+    assert _lib.layout(ps)[1] != key
+    ps[1].grad = torch.nn.Parameter(torch.zeros(3))  # as plain as a tensor
+    assert isinstance(_lib.layout(ps)[1], bytes)

@@ -24,8 +24,9 @@ void put_tensor(std::string& s, const at::Tensor& t) {
 }
 
 // layout(params) -> (active, key): the entries of the list that have a
-// gradient, and their layouts as bytes.  None when an entry is neither a plain
-// Tensor nor a plain Parameter (a subclass may define its own attributes).
+// gradient, and their layouts as bytes.  None when an entry or its gradient is
+// neither a plain Tensor nor a plain Parameter (a subclass may define its own
+// attributes).
 PyObject* layout(PyObject*, PyObject* params) {
     HANDLE_TH_ERRORS
     if (!PyList_CheckExact(params)) Py_RETURN_NONE;
@@ -40,6 +41,9 @@ PyObject* layout(PyObject*, PyObject* params) {
         const at::Tensor& t = THPVariable_Unpack(p);
         const at::Tensor g = t.grad();
         if (!g.defined()) continue;
+        THPObjectPtr gradient(THPVariable_Wrap(g));
+        if (!gradient) return nullptr;
+        if (!THPVariable_CheckExact(gradient.get())) Py_RETURN_NONE;
         if (PyList_Append(active.get(), p) != 0) return nullptr;
         put(key, reinterpret_cast<int64_t>(p));
         put_tensor(key, t);
