@@ -1,9 +1,13 @@
 """The native layout key of launch plans (csrc/layout.cpp): it changes exactly
 when the attribute-by-attribute key (``_lib.layout_key``) does."""
 
+import sys
+import types
+
+import pytest
 import torch
 
-from triton_muon_adamw import _lib
+from triton_muon_adamw import _build, _lib
 
 
 def _params():
@@ -98,3 +102,37 @@ def test_layout_of_a_subclass_gradient():
     assert _lib.layout(ps)[1] != key
     ps[1].grad = torch.nn.Parameter(torch.zeros(3))  # as plain as a tensor
     assert isinstance(_lib.layout(ps)[1], bytes)
+
+
+@pytest.mark.parametrize("module", [None, types.SimpleNamespace(torch_version="0.0.1", layout=lambda params: 1 / 0)],
+                         ids=["missing", "of_another_torch"])
+def test_layout_without_the_native_module(monkeypatch, module):
+    """Built for another Python or torch, or not built: the same parameters and
+    keys that follow the same changes, after one warning."""
+    import triton_muon_adamw
+
+    monkeypatch.setattr(_lib, "_layout", None)
+    monkeypatch.setitem(sys.modules, "triton_muon_adamw._layout", module)  # None: the import fails
+    monkeypatch.delattr(triton_muon_adamw, "_layout", raising=False)
+    if module is not None:
+        monkeypatch.setattr(triton_muon_adamw, "_layout", module, raising=False)
+    ps = _params()
+    with pytest.warns(RuntimeWarning, match="launch plans are compared in Python") as seen:
+        active, key = _lib.layout(ps)
+        assert _lib.layout(ps)[1] == key
+    assert len(seen) == 1
+    assert [id(p) for p in active] == [id(p) for p in ps[:4]] and key == tuple(_lib.layout_key(p) for p in ps[:4])
+    ps[0].grad = ps[0].grad.clone()
+    assert _lib.layout(ps)[1] != key
+
+
+def test_build_without_a_compiler_for_the_native_module(monkeypatch, tmp_path):
+    """The kernels' build goes on, and no module of an older build is left to be loaded."""
+    stale = tmp_path / "_layout.so"
+    stale.write_bytes(b"")
+    monkeypatch.setattr(_build, "LAYOUT_PATH", stale)
+    for cxx in (str(tmp_path / "no-such-compiler"), "false"):
+        monkeypatch.setenv("CXX", cxx)
+        with pytest.warns(RuntimeWarning, match="was not built"):
+            _build._build_layout(verbose=False)
+        assert not stale.exists()

@@ -9,6 +9,7 @@
 #include <torch/csrc/autograd/python_variable.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/utils/object_ptr.h>
+#include <torch/version.h>
 
 #include <string>
 
@@ -65,5 +66,7 @@ PyModuleDef kModule = {PyModuleDef_HEAD_INIT, "_layout", nullptr, -1, kMethods, 
 }  // namespace
 
 PyMODINIT_FUNC PyInit__layout() {
-    return PyModule_Create(&kModule);
+    THPObjectPtr m(PyModule_Create(&kModule));
+    if (!m || PyModule_AddStringConstant(m.get(), "torch_version", TORCH_VERSION) != 0) return nullptr;
+    return m.release();
 }

@@ -12,6 +12,7 @@ from __future__ import annotations
 
 import ctypes
 import threading
+import warnings
 from ctypes import POINTER, c_char_p, c_double, c_float, c_int, c_int32, c_int64, c_size_t, c_void_p
 from pathlib import Path
 
@@ -206,21 +207,33 @@ def layout_key(p: torch.Tensor) -> tuple:
 _layout = None
 
 
+def _load_layout():
+    """The native reader of layouts; one that reads nothing (with a warning)
+    where this installation has none built for this Python and torch."""
+    try:
+        from . import _layout as module
+        why = module.torch_version != torch.__version__.split("+")[0] and f"built with torch {module.torch_version}"
+    except ImportError as e:
+        why = str(e)
+    if not why:
+        return module.layout
+    warnings.warn(f"triton_muon_adamw._layout cannot be used ({why}): launch plans are compared in Python, about 1 us "
+                  "a parameter and step. Run __graft_entry__.build() (or python -m triton_muon_adamw._build).",
+                  RuntimeWarning, stacklevel=4)
+    return lambda params: None
+
+
 def layout(params) -> tuple[list, object]:
     """``(active, key)``: the parameters that have a gradient, and what a launch
     plan of them assumes (``layout_key`` of each), in a form that compares
     equal exactly while none of it changed.  Read natively
     (``csrc/layout.cpp``) from a list of plain tensors and parameters; tensor
-    subclasses and other sequences attribute by attribute."""
+    subclasses and other sequences, and all where there is no native reader,
+    attribute by attribute."""
     global _layout
     if _layout is None:
-        try:
-            from . import _layout as module
-        except ImportError as e:
-            raise RuntimeError("_layout is not built; run __graft_entry__.build() "
-                               "(or python -m triton_muon_adamw._build)") from e
-        _layout = module
-    found = _layout.layout(params)
+        _layout = _load_layout()
+    found = _layout(params)
     if found is None:
         active = [p for p in params if p.grad is not None]
         found = active, tuple(layout_key(p) for p in active)
