@@ -23,3 +23,13 @@ def gpu():
     if not torch.cuda.is_available():
         pytest.fail("this test needs a ROCm GPU")
     return torch.device("cuda:0")
+
+
+@pytest.fixture
+def staged(monkeypatch):
+    """HipMuon and muon_step take the LDS-staged kernels whatever the sizes (small
+    groups would go out on the direct path)."""
+    from triton_muon_adamw.muon import hip_muon
+
+    monkeypatch.setattr(hip_muon, "direct_pays", lambda *_: False)
+    monkeypatch.setattr(hip_muon, "direct_set_pays", lambda *_: False)

@@ -251,7 +251,7 @@ def planner(monkeypatch):
     monkeypatch.setattr(torch.cuda, "get_device_properties", lambda dev: props)
     monkeypatch.setattr(_lib, "require_gpu_tensor", lambda t, name: None)
     monkeypatch.setattr(_lib, "raw_stream", lambda dev: 0)
-    monkeypatch.setattr(_lib, "side_streams", lambda dev, n: [streams.append(n) or f"side{i}" for i in range(n)])
+    monkeypatch.setattr(_lib, "side_streams", lambda dev, n: streams.append(n) or [f"side{i}" for i in range(n)])
 
     def plan(shapes, limit=None, **attributes):
         params = [torch.nn.Parameter(torch.zeros(s)) for s in shapes]
@@ -288,6 +288,73 @@ def test_launches_keep_to_the_workspace_limit(planner, limit_mib, in_order):
             assert need <= limit or not x.direct and x.n == 1 and one == {need}
     if not in_order and limit is None:  # 36 matrices, one launch
         assert [(x.n, x.direct, x.lane) for x in opt._launches] == [(36, True, None)]
+
+
+def test_streams_for_staged_classes_only(planner):
+    """Classes that go out together on the caller's stream make no side streams
+    (a thread keeps those it makes); staged classes run on the ones made."""
+    opt = planner([(256, 1024)] * 4 + [(256, 768)] * 2 + [(256, 256)] * 2)
+    assert opt._concurrent and [(x.n, x.direct, x.lane) for x in opt._launches] == [(8, True, None)]
+    assert planner.streams == [] and opt._lanes == {}
+    opt = planner([(1024, 2048), (2048, 4096), (4096, 4096), (4096, 1024)])
+    assert opt._concurrent and not any(x.direct for x in opt._launches)
+    lanes = [x.lane for x in opt._launches]
+    assert planner.streams == [2] and lanes[0] is None and set(lanes[1:]) == {"side0", "side1"}
+    assert len({x.ws_key for x in opt._launches}) == 4
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("how", ["current", "side", "graph"])
+def test_merged_classes_equal_staged_in_order(gpu, monkeypatch, how):
+    """Shape classes that go out as one direct launch, on the caller's stream:
+    the bits of staged classes one after another, also under a side stream and
+    in a graph that is replayed between eager work."""
+    shapes = [(256, 512)] * 3 + [(512, 256)] * 2 + [(384, 384)] * 2 + [(128, 640), (10, 517)]
+    start = _make(shapes, gpu, F32, F32, 0, False)
+    grads = [_make(shapes, gpu, F32, F32, 0, False)[i][1] * (1 + i / 7) for i in range(len(shapes))]
+
+    def optimizer():
+        params = [torch.nn.Parameter(p.clone()) for p, _, _, _ in start]
+        opt = hip_muon.HipMuon(params, lr=2e-2, coeffs=COEFFS)
+        for p, g, (_, _, m, _) in zip(params, grads, start):
+            p.grad = g.clone()
+            opt.momentum[p].copy_(m)
+        return params, opt
+
+    params, opt = optimizer()
+    rparams, ropt = optimizer()
+    ropt.concurrent_flops_limit = 0.0
+
+    def reference_step():
+        with monkeypatch.context() as m:
+            m.setattr(hip_muon, "direct_pays", lambda *_: False)
+            ropt.step()
+        assert not any(x.direct for x in ropt._launches)
+
+    def compare():
+        torch.cuda.synchronize()
+        for p, q in zip(params, rparams):
+            assert torch.equal(p, q) and torch.equal(opt.momentum[p], ropt.momentum[q])
+
+    opt.step()
+    assert opt._concurrent and [(x.n, x.direct, x.lane) for x in opt._launches] == [(9, True, None)]
+    reference_step()
+    compare()
+    if how == "graph":
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            opt.step()
+    side = torch.cuda.Stream(device=gpu) if how == "side" else torch.cuda.current_stream(gpu)
+    for i in range(4):
+        for p, q in zip(params, rparams):  # other gradients in the same buffers
+            p.grad.mul_(-1.25)
+            q.grad.mul_(-1.25)
+        side.wait_stream(torch.cuda.current_stream(gpu))
+        with torch.cuda.stream(side):
+            graph.replay() if how == "graph" else opt.step()
+        torch.cuda.current_stream(gpu).wait_stream(side)
+        reference_step()
+        compare()
 
 
 # ---- Standalone products ----------------------------------------------------

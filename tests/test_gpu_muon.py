@@ -284,7 +284,7 @@ CONCURRENT_SETS = {
 
 @pytest.mark.parametrize("classes", sorted(CONCURRENT_SETS))
 @pytest.mark.parametrize("on_side_stream", [False, True])
-def test_concurrent_classes_equal_in_order(gpu, on_side_stream, classes):
+def test_concurrent_classes_equal_in_order(gpu, staged, on_side_stream, classes):
     """Shape classes on their own streams (small steps) give the same bits as one after another,
     also when the caller steps on a non-default stream and reads the result there."""
     shapes = CONCURRENT_SETS[classes]
@@ -307,7 +307,8 @@ def test_concurrent_classes_equal_in_order(gpu, on_side_stream, classes):
                 opt.step()
             assert opt._concurrent == (limit > 0)
             if limit > 0:
-                side = {id(st) for st in opt._lanes.values() if st is not None}
+                side = {id(x.lane) for x in opt._launches if x.lane is not None}
+                assert sum(x.lane is None for x in opt._launches) == 1
                 assert len(side) == (3 if classes == "five_classes" else 2)
             out = [q.detach().clone() for q in params] + [opt.momentum[q].clone() for q in params]
         torch.cuda.current_stream(gpu).wait_stream(stream)

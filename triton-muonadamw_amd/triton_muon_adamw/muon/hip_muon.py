@@ -731,13 +731,17 @@ class HipMuon:
                 c.direct = together if concurrent else fits[c] and direct_pays(c.m, c.n_, c.n, cus, self.steps)
                 c.ws_bytes = (_direct_workspace_bytes(c.arr, c.n, self.steps) if c.direct
                               else _workspace_bytes(c.n, c.m, c.n_, self.steps))
+        # Concurrent classes, longest first (a class's own launches keep their
+        # order: stable sort), the staged ones on streams.  Direct ones need
+        # none: one launch on the caller's holds them all (up to
+        # MUON_DIRECT_MAX matrices).
         self._lanes = {}
-        if concurrent:  # longest class first; a class's own launches keep their order (stable sort)
-            cus = {d: torch.cuda.get_device_properties(d).multi_processor_count for d in dict.fromkeys(c.device for c in calls)}
-            self._lanes, times = _lanes(calls, self.steps, cus)
+        if concurrent:
+            cus = {c.device: torch.cuda.get_device_properties(c.device).multi_processor_count for c in calls}
+            self._lanes, times = _lanes([c for c in calls if not c.direct], self.steps, cus)
+            for key in {(c.device, c.group) for c in calls if c.direct}:
+                times[key] = _class_time(calls, key, self.steps, cus[key[0]])
             calls.sort(key=lambda c: -times[(c.device, c.group)])
-        # The launches.  Concurrent direct classes need no streams: one launch
-        # on the caller's holds them all (up to MUON_DIRECT_MAX matrices).
         launches, need = [], {}
         for dev in dict.fromkeys(c.device for c in calls):
             mine = [c for c in calls if c.device == dev]
