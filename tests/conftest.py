@@ -33,3 +33,10 @@ def staged(monkeypatch):
 
     monkeypatch.setattr(hip_muon, "direct_pays", lambda *_: False)
     monkeypatch.setattr(hip_muon, "direct_set_pays", lambda *_: False)
+
+
+@pytest.fixture(params=["chosen", "staged"])
+def path(request):
+    """The kernels that the sizes choose (for small sets the direct path), and the staged ones."""
+    if request.param == "staged":
+        request.getfixturevalue("staged")

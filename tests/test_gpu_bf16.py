@@ -90,7 +90,7 @@ def test_muon_bf16_vs_oracle(gpu, shape):
 
 @pytest.mark.parametrize("shapes,tile", [([(1024, 2048)] * 4 + [(2048, 1024)] * 4, 256),
                                          ([(768, 3072)] * 6 + [(3072, 768)] * 6, 192)])
-def test_muon_bf16_params_batched_equal_single(gpu, shapes, tile):
+def test_muon_bf16_params_batched_equal_single(gpu, staged, shapes, tile):
     """bf16 parameters through the batched APPLY epilogues of the 256 x 256
     tile and of the 128 x 192 update tile (the group of 8 or 12) against each
     matrix stepped alone (128 x 128 tiles): the same products in the same

@@ -280,13 +280,13 @@ def test_steps_do_not_synchronise(gpu):
 
 
 @pytest.mark.parametrize("in_order", [True, False])
-def test_steps_under_a_side_stream(gpu, in_order):
+def test_steps_under_a_side_stream(gpu, path, in_order):
     """Steps taken with a side stream current (every other step), with new
     gradient tensors each step so that the AdamW table is re-packed and the
     launch groups rebuilt while earlier launches may still be queued, give the
     same parameters bit for bit as steps on the default stream.  ``in_order``
     runs the Muon shape classes in order on the caller's stream (the path of
-    large steps) instead of on forked side streams."""
+    large steps) instead of on forked side streams (where they are staged)."""
     a, b = _params(gpu), _params(gpu)
     opt_a = MuonAdamW(_split(a), muon_config=MC, adam_config=AC, parameter_split="explicit")
     opt_b = MuonAdamW(_split(b), muon_config=MC, adam_config=AC, parameter_split="explicit")
@@ -315,15 +315,15 @@ def test_steps_under_a_side_stream(gpu, in_order):
 
 
 @pytest.mark.parametrize("in_order", [True, False])
-def test_graph_captured_step_replays_like_eager_steps(gpu, in_order):
+def test_graph_captured_step_replays_like_eager_steps(gpu, path, in_order):
     """``capturable=True``: one eager step, then a step captured with
     ``torch.cuda.graph`` and replayed three times (new gradients copied into the
     static ``.grad`` tensors before each replay, eager steps of a twin
     optimizer and a synchronisation between replays) gives the parameters,
     moments and momentum of four eager steps bit for bit, each replay checked;
     the device step counter reads 4.  ``in_order``: Muon shape classes in
-    order on the capture stream, else forked onto side streams inside the
-    graph."""
+    order on the capture stream, else (where they are staged) forked onto side
+    streams inside the graph."""
     a, b = _params(gpu), _params(gpu)
     opt_a = MuonAdamW(_split(a), muon_config=MC, adam_config=AC, parameter_split="explicit", capturable=True)
     opt_b = MuonAdamW(_split(b), muon_config=MC, adam_config=AC, parameter_split="explicit")

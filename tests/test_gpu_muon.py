@@ -112,11 +112,11 @@ RAGGED_SHAPES = [(300, 1000), (1000, 300), (1000, 300), (200, 520), (520, 200)]
 
 
 @pytest.mark.parametrize("nesterov,ns_steps", [(True, 5), (False, 5), (True, 1), (True, 0), (True, 2)])
-def test_muon_step_vs_oracle(gpu, nesterov, ns_steps):
+def test_muon_step_vs_oracle(gpu, path, nesterov, ns_steps):
     _check_vs_oracle(gpu, SMALL_SHAPES, nesterov, ns_steps)
 
 
-def test_ragged_multi_tile_vs_oracle(gpu):
+def test_ragged_multi_tile_vs_oracle(gpu, path):
     _check_vs_oracle(gpu, RAGGED_SHAPES, True, 5)
 
 
@@ -154,7 +154,7 @@ def _check_vs_oracle(gpu, shapes, nesterov, ns_steps):
         np.testing.assert_allclose(got, oracle.muon.fma32(-slr, upd, ps[i].numpy() * keep), rtol=0, atol=1e-7)
 
 
-def test_batched_equals_single(gpu):
+def test_batched_equals_single(gpu, path):
     shapes = [(256, 512)] * 3 + [(512, 256)] * 2
     ps, gs, ms, params, opt = _run_muon(shapes, gpu, seed=4)
     singles = []
@@ -171,7 +171,7 @@ def test_batched_equals_single(gpu):
         assert torch.equal(a.detach(), b.detach())
 
 
-def test_parameter_listed_twice_steps_twice(gpu):
+def test_parameter_listed_twice_steps_twice(gpu, path):
     """A matrix listed twice gets two Muon updates in sequence (momentum and
     parameter), as the reference's per-parameter loop gives it
     (triton_muon.py:415-448, state keyed by the parameter): its second
@@ -197,7 +197,7 @@ def test_parameter_listed_twice_steps_twice(gpu):
         assert torch.equal(opt.momentum[p], o.momentum[q])
 
 
-def test_rect_tile_does_not_change_the_bits(gpu):
+def test_rect_tile_does_not_change_the_bits(gpu, staged):
     """Twelve 768 x 3072 matrices (the tall and the wide orientation) in one
     launch group run their updates on 128 x 192 tiles (1152 tiles, at least
     two rounds); each alone runs them on 128 x 128 tiles.  Every output
@@ -219,7 +219,7 @@ def test_rect_tile_does_not_change_the_bits(gpu):
         step_fn()
         _lib.prof_stop()
         return {(r["kernel"].split(":")[1], r["variant"] // 8) for r in _lib.prof_collect()
-                if r["kernel"].startswith("ns_gemm")}
+                if r["kernel"].startswith("ns_gemm_kernel")}
 
     assert tiles_of(opt.step) == {("gram", 128), ("poly", 128), ("update", 192), ("apply", 192)}
     assert tiles_of(lambda: [o.step() for _, o in singles]) == {("gram", 128), ("poly", 128), ("update", 128),
@@ -233,11 +233,11 @@ def test_rect_tile_does_not_change_the_bits(gpu):
         assert torch.equal(opt.momentum[a], o.momentum[b])
 
 
-def test_tile_edge_does_not_change_the_bits(gpu):
+def test_tile_edge_does_not_change_the_bits(gpu, staged):
     """Eight 1024 x 2048 matrices in one launch group run on 256-wide tiles
     (m >= 1024 and 8 matrices) with lower-triangle A and B; each alone runs
-    its Gram and polynomial on 128-wide tiles with mirrored A and B (the
-    updates take 256-wide tiles from m = 1024 either way).  Every output
+    its Gram and polynomial on 128-wide tiles with mirrored A and B (its
+    updates too: 32 256-wide tiles run as 128-wide quarters).  Every output
     element sums the same products in the same order under either tile and
     layout, so parameters and momenta agree bit for bit (two steps)."""
     from triton_muon_adamw import _lib
@@ -256,13 +256,13 @@ def test_tile_edge_does_not_change_the_bits(gpu):
         step_fn()
         _lib.prof_stop()
         return {(r["kernel"].split(":")[1], r["variant"] // 8) for r in _lib.prof_collect()
-                if r["kernel"].startswith("ns_gemm")}
+                if r["kernel"].startswith("ns_gemm_kernel")}
 
     assert tiles_of(opt.step) == {("gram", 256), ("poly", 256), ("update", 256), ("apply", 256)}
     assert [c.n for c in opt._calls] == [8]
-    # alone: 128-wide Gram and polynomial, 256-wide updates (m = 1024)
-    assert tiles_of(lambda: [o.step() for _, o in singles]) == {("gram", 128), ("poly", 128), ("update", 256),
-                                                                 ("apply", 256)}
+    # alone: 128-wide Gram and polynomial, updates as quarters of 32 256-wide tiles
+    assert tiles_of(lambda: [o.step() for _, o in singles]) == {("gram", 128), ("poly", 128), ("update", 128),
+                                                                 ("apply", 128)}
     opt.step()
     for q, o in singles:
         o.step()
@@ -330,8 +330,8 @@ SWEEP = [(3, (200, 520)), (5, (700, 260)), (1, (129, 4000)), (8, (1024, 1300)), 
 
 
 @pytest.mark.parametrize("count,shape", SWEEP)
-def test_group_sweep_vs_torch(gpu, count, shape):
-    """A launch group of ``count`` matrices of ``shape``: every matrix's update
+def test_group_sweep_vs_torch(gpu, staged, count, shape):
+    """A staged launch group of ``count`` matrices of ``shape``: every matrix's update
     (recovered from the parameter change, in float64) against torch's
     Newton-Schulz (``torch.optim._muon._zeropower_via_newtonschulz``) of the
     same Nesterov blend, relative Frobenius error <= 1e-2."""
@@ -358,7 +358,7 @@ def test_group_sweep_vs_torch(gpu, count, shape):
 
 
 @pytest.mark.parametrize("shape", [(200, 520), (520, 200)])
-def test_zero_gradient_members_only_decay(gpu, shape):
+def test_zero_gradient_members_only_decay(gpu, path, shape):
     """A launch group whose members 1 and 3 have zero gradient and zero
     momentum: X = 0, so ||X|| = 0 and X / max(||X||, eps) = 0 (torch's
     clamp), the Newton-Schulz iterate stays 0 and the parameter only decays,
@@ -469,7 +469,7 @@ def _orthogonal_signs(rows, cols, rng, order=4096):
 
 @pytest.mark.parametrize("count,shape,order", [(16, (1024, 4096), 4096), (1, (14336, 4096), 4096),
                                                (16, (512, 2304), 2048)])
-def test_ns_exact_on_orthogonal_rows(gpu, count, shape, order):
+def test_ns_exact_on_orthogonal_rows(gpu, staged, count, shape, order):
     """The whole Newton-Schulz pipeline on inputs where every product is exact
     in any summation order, so the result is known bit for bit.
 
