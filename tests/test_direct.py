@@ -426,6 +426,45 @@ def test_ns_outputs_of_any_kind(gpu):
         hip_muon.solve_ns_kernel_1(flat[1:].view(128, 128), torch.empty((128, 128), dtype=BF16, device=gpu))
 
 
+def test_ns_direct_leaves_other_tensors_to_the_copy(monkeypatch):
+    """Outputs and inputs of a subclass (their own copy_ runs) and calls in
+    forward mode (copy_ clears the output's tangent) do not go past it."""
+    class Sub(torch.Tensor):
+        pass
+
+    monkeypatch.setattr(torch.cuda, "get_device_properties",
+                        lambda dev: types.SimpleNamespace(multi_processor_count=256))
+    reached = []
+    monkeypatch.setattr(hip_muon, "ns_direct_pays", lambda *_: reached.append(1))  # None: not direct
+    x, s, out = torch.zeros(96, 200, dtype=BF16), torch.zeros(96, 96, dtype=BF16), torch.zeros(96, 200, dtype=BF16)
+
+    def call(x=x, s=s, out=out):
+        del reached[:]
+        assert not hip_muon._ns_direct(2, x, s, out, 1.0, 0.0, 0.0)
+        return bool(reached)
+
+    assert call() and call(x=torch.nn.Parameter(x)) and call(out=torch.nn.Parameter(out, requires_grad=False))
+    assert not call(out=out.as_subclass(Sub)) and not call(x=x.as_subclass(Sub)) and not call(s=s.as_subclass(Sub))
+    with torch.autograd.forward_ad.dual_level():
+        assert not call(out=torch.autograd.forward_ad.make_dual(out, torch.ones_like(out)))
+    assert call()
+
+
+@pytest.mark.gpu
+def test_ns_output_with_a_tangent(gpu):
+    """Forward mode: writing the output clears its tangent, as any in-place copy of a constant does."""
+    x, s = _ns_inputs(96, 200, gpu)
+    for op in range(4):
+        shape = (96, 96) if op < 2 else (96, 200)
+        ref = torch.empty(shape, dtype=BF16, device=gpu)
+        _ns_call(op, x, s, ref)
+        with torch.autograd.forward_ad.dual_level():
+            out = torch.autograd.forward_ad.make_dual(torch.zeros_like(ref), torch.ones_like(ref))
+            _ns_call(op, x, s, out)
+            primal, tangent = torch.autograd.forward_ad.unpack_dual(out)
+            assert torch.equal(primal, ref) and (tangent is None or not tangent.any()), op
+
+
 def test_ns_direct_rejects_before_hip():
     NULL, SHAPE, ALIGN, WS, HYPER, ALIAS = -1, -4, -5, -6, -7, -9
     lib = _lib.load()

@@ -41,6 +41,7 @@ from typing import Literal
 
 import torch
 import torch.nn as nn
+from torch.autograd import forward_ad
 
 from .. import _lib
 
@@ -207,6 +208,7 @@ def _check_bf16_2d(x: torch.Tensor, name: str) -> None:
         raise TypeError(f"{name} must be bfloat16 (got {x.dtype})")
 
 
+_PLAIN = (torch.Tensor, nn.Parameter, type(None))  # no attributes or copies of their own
 _NS_GRAM, _NS_POLY, _NS_UPDATE, _NS_STEP = range(4)  # MAMW_NS_*
 
 
@@ -252,9 +254,12 @@ def _ns_direct(op: int, X: torch.Tensor, S, out: torch.Tensor, a: float, b: floa
     """The product on the direct path, straight into ``out``; False where it
     stays with the padded, staged one: inputs or an output that are not plain
     contiguous bf16 matrices of the right shape on one device (copies there
-    handle any strides, types and broadcasts, and refuse what autograd must
-    refuse), 16-byte misaligned inputs (which it refuses unless it pads them),
-    and sizes where it is the faster one."""
+    handle any strides, types, subclasses and broadcasts, and refuse what
+    autograd must refuse), an output with a forward-mode tangent (which the
+    copy clears), 16-byte misaligned inputs (which it refuses unless it pads
+    them), and sizes where it is the faster one."""
+    if any(type(t) not in _PLAIN for t in (X, S, out)) or forward_ad.unpack_dual(out).tangent is not None:
+        return False
     m, n = X.shape
     shape = (m, m) if op in (_NS_GRAM, _NS_POLY) else (m, n)
     if (m < 1 or n < 1 or out.dtype != torch.bfloat16 or out.shape != shape or out.device != X.device
