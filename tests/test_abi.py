@@ -5,6 +5,7 @@ fake addresses: validation never dereferences them."""
 
 import ctypes
 import re
+import subprocess
 from pathlib import Path
 
 import pytest
@@ -358,6 +359,38 @@ def test_ns_blocks_reject_overlapping_buffers():
     assert lib.mamw_ns_update(B, out, XT, out, B, 1, m, n, 3.44, None) == ALIAS
     assert lib.mamw_ns_update(B, out, XT, out, XT + 4096, 1, m, n, 3.44, None) == ALIAS
     assert lib.mamw_ns_update(B, out, XT, out, out + 2 * m * n - 16, 1, m, n, 3.44, None) == ALIAS
+
+
+def test_profiler_without_a_second_event(tmp_path):
+    """prof_take with one event left to be had: no record, and neither event is
+    handed out (the first is free again).  Host code with a stub hipEventCreate."""
+    from triton_muon_adamw import _build
+
+    main = tmp_path / "main.cpp"
+    main.write_text("""
+#include <hip/hip_runtime_api.h>
+#include "mamw_launch.h"
+static int left = 1;
+extern "C" hipError_t hipEventCreate(hipEvent_t* e) {
+    if (left == 0) return hipErrorOutOfMemory;
+    --left;
+    *e = reinterpret_cast<hipEvent_t>(8);
+    return hipSuccess;
+}
+int main() {
+    hipEvent_t a = nullptr, b = nullptr;
+    if (mamw_prof_start() != 0) return 2;
+    if (mamw::prof_take(&a, &b) || a || b) return 1;
+    left = 1;  // with the one given back, two
+    return mamw::prof_take(&a, &b) && a && b ? 0 : 3;
+}
+""")
+    exe = tmp_path / "main"
+    cmd = [_build._hipcc(), *_build.COMMON_FLAGS, "-x", "c++", "-I/opt/rocm/include", "-D__HIP_PLATFORM_AMD__",
+           str(main), str(_build.CSRC / "prof.cpp"), "-o", str(exe)]
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    assert res.returncode == 0, res.stderr
+    assert subprocess.run([str(exe)]).returncode == 0
 
 
 def test_profiler_without_launches():

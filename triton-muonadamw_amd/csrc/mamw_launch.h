@@ -39,7 +39,7 @@ enum KernelId : int32_t {
 };
 
 // Returns true and two events when profiling is on (and not suspended on
-// this thread).
+// this thread); else false, start and stop as they were.
 bool prof_take(hipEvent_t* start, hipEvent_t* stop);
 
 // While one of these lives, launches on this thread take no profiler events

@@ -68,13 +68,14 @@ bool prof_take(hipEvent_t* start, hipEvent_t* stop) {
     if (g_suspended) return false;
     std::lock_guard<std::mutex> lk(g_mu);
     if (!g_on) return false;
-    *start = take_event();
-    *stop = take_event();
-    if (!*start || !*stop) {
-        if (*start) keep_free(*start);
-        if (*stop) keep_free(*stop);
+    const hipEvent_t e0 = take_event(), e1 = take_event();
+    if (!e0 || !e1) {
+        if (e0) keep_free(e0);
+        if (e1) keep_free(e1);
         return false;
     }
+    *start = e0;
+    *stop = e1;
     return true;
 }
 
