@@ -241,7 +241,8 @@ int mamw_muon_step_amp(const mamw_muon_matrix* mats, int batch, double lr,
  * output tile (muon_direct.hip).  Results, bit for bit, are those of
  * mamw_muon_step / mamw_muon_step_amp on each matrix; grad_scale and found_inf
  * as there (NULL: a plain step).  ns_steps >= 1; a matrix padded to multiples
- * of 64 holds at most 2^26 elements (MAMW_ERR_SHAPE beyond).  The workspace
+ * of 128 in both dimensions holds at most 2^26 elements (MAMW_ERR_SHAPE
+ * beyond; so 1 x 2^19 is taken and 1 x 2^20 refused).  The workspace
  * (256-byte aligned, mamw_muon_direct_workspace_bytes, which reads the rows
  * and cols only) also keeps X beside its transpose, so it is larger than
  * mamw_muon_workspace_bytes.                                                 */

@@ -172,7 +172,8 @@ def test_direct_rejects_before_hip():
     assert _bytes(_mats(ok), 0)[0] == COUNT and _bytes(_mats([(4, 4)] * 65), 65)[0] == COUNT
     assert _bytes(_mats(ok), 2, steps=0)[0] == HYPER and _bytes(_mats(ok), 2, steps=100)[0] == HYPER
     assert _bytes(_mats([(0, 4)]), 1)[0] == SHAPE and _bytes(_mats([(8192, 8256)]), 1)[0] == SHAPE
-    assert _bytes(_mats([(1, 1 << 20)]), 1)[0] == SHAPE  # too many prep units for one block to sum
+    # padded to 128: 2^26 elements, and twice as many (too many prep units for one block to sum)
+    assert _bytes(_mats([(1, 1 << 19)]), 1)[0] == 0 and _bytes(_mats([(1, 1 << 20)]), 1)[0] == SHAPE
     assert _step(_mats(ok), 2, ws_bytes=need - 1) == WS and _step(_mats(ok), 2, ws=None) == WS
     assert _step(_mats(ok), 2, ws=(1 << 45) + 64) == WS
     for field, value, code in (("param", None, NULL), ("flags", 4, HYPER), ("momentum", (1 << 45) + 256, ALIAS),

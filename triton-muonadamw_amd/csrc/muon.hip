@@ -1505,9 +1505,9 @@ hipError_t launch_gemm(int tile, const GemmArgs& g, const MuonBatchDescs& d, int
     // a round (below that m the 256 tile is taken only by groups that measured
     // faster with it; an update's last 65 to 128 tiles after full rounds stay).
     // The storage stays that of the 256-wide tiles, and each element its sum.
-    // Steps, whole rounds -> split: 2048 x 2048 632 -> 355 us, 4096 x 2048 799
-    // -> 557, two 4096 x 4096 (272 symmetric tiles) 2850 -> 2607, 26 of 1024 x
-    // 4096 2805 -> 2704.
+    // Steps, whole rounds -> split: 2048 x 2048 636 -> 347 us, 4096 x 2048 799
+    // -> 509, two 4096 x 4096 (272 symmetric tiles) 2815 -> 2567, 26 of 1024 x
+    // 4096 2762 -> 2654.
     constexpr int kRound = kXcds * kXcdSlots;
     const int full = total / kRound * kRound, tail = total - full;
     const bool large = g.tiles_m >= 8;

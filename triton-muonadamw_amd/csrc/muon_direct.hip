@@ -10,9 +10,9 @@
 // Every output element sums the same products in the same order as there (one
 // v_mfma_f32_32x32x16_bf16 chain, k ascending), so the results are the same
 // bits.  Measured in the step, staged -> direct: one 3072 x 768 matrix, Gram
-// 28.5 -> 8.8 us, polynomial 10.3 -> 4.5, update 10.7 -> 11.4, step 268 -> 151;
-// two 512 x 2048, Gram 18 -> 6, polynomial 8 -> 4, update 9.9 -> 9, step 198 ->
-// 117.  What is left of a small launch is latency: 1.5 us for an empty kernel,
+// 28.6 -> 8.9 us, polynomial 9.9 -> 4.3, update 10.5 -> 10.6, step 269 -> 143;
+// two 512 x 2048, Gram 17.8 -> 6.0, polynomial 7.6 -> 3.9, update 9.5 -> 8.6,
+// step 198 -> 108.  What is left of a small launch is latency: 1.5 us for an empty kernel,
 // then the arguments, the operands (written by other XCDs, so past the L2) and
 // the stores, one after the other.  A larger one is bound by the L2's operand
 // traffic (26 TB/s fits 460 measured steps), which the staged tiles halve: the
@@ -436,7 +436,7 @@ __global__ __launch_bounds__(64, 2) void direct_gemm_kernel(char* ws, const Dire
     }
 
     // Apply: a tile that lies inside the parameter loads its elements now, so
-    // that their HBM latency passes under the operands' (13.8 -> see below).
+    // that their HBM latency passes under the operands'.
     // Lane: column x = tx T + 32 c + lane % 32, rows 4 (lane / 32) + constants,
     // whose offsets ride in the scalar offset.
     const bool bf = MODE == DM_APPLY && (d.flags & MAMW_BF16_PARAM) != 0;
@@ -649,8 +649,8 @@ __global__ __launch_bounds__(64, 2) void direct_gemm_kernel(char* ws, const Dire
     uint16_t* const along = MODE == DM_GRAM ? A : MODE == DM_POLY ? B : X;
     // Stores write through the L2 (kStoreThrough): the tiles of a small launch
     // end together, and what is still dirty in the L2s is written back before
-    // the next launch may begin (2 x 512 x 2048 step 115 -> 109 us, 4 x 768 x
-    // 768 160 -> 152, 2048 x 2048 325 -> 311).
+    // the next launch may begin (steps without -> with: two 512 x 2048 113 ->
+    // 108 us, four 768 x 768 159 -> 152, 2048 x 2048 319 -> 308).
     const __amdgpu_buffer_rsrc_t r_across = rsrc(across, int64_t(xrows) * (SYM ? mp : yrows) * 2);
     const __amdgpu_buffer_rsrc_t r_along = rsrc(along, int64_t(yrows) * (SYM ? mp : xrows) * 2);
 #pragma unroll

@@ -84,11 +84,14 @@ def _direct_workspace_bytes(arr, count: int, ns_steps: int) -> int:
 # the direct path (mamw_muon_direct_step, one wavefront per 32- or 64-wide
 # tile), the same bits either way.  Both times are estimated in microseconds
 # per step (five iterations) with constants fitted to 460 measured pairs on one
-# MI355X: 16 <= m <= 4096, n up to 16 m, 1 to 32 matrices; standard error 6%
-# each, and the cheaper path was named wrongly with a loss over 6% in 5 of
-# them.  Measured on both sides (staged / direct): 512 x 2048 one matrix 194 /
-# 101, two 198 / 116, eight 238 / 228, sixteen 328 / 374; 768 x 3072 one 268 /
-# 151, eight 438 / 518; 2048 x 2048 one 632 / 331, four 795 / 1088.
+# MI355X (16 <= m <= 4096, n up to 16 m, 1 to 32 matrices), before the direct
+# stores were written through and the staged last rounds split, which the
+# staged estimate has a term for.  Against 130 pairs of the kernels as they are
+# now: rms error 9% staged, 11% direct; the choice lost over 6% (at most 27%) in
+# 12 of them, each a staged launch that the direct path would have beaten.
+# Measured on both sides (staged / direct): 512 x 2048 one matrix 195 / 96, two
+# 198 / 109, eight 240 / 219, sixteen 339 / 372; 768 x 3072 one 268 / 143, eight
+# 443 / 512; 2048 x 2048 one 347 / 307, four 782 / 1036.
 
 def _staged_product_us(tile: int, tiles: int, k: int, cus: int, split: bool, sym: bool = False,
                        large: bool = False) -> float:
@@ -159,7 +162,8 @@ def _direct_fits(m: int, n: int, ns_steps: int) -> bool:
 def direct_pays(rows: int, cols: int, count: int, cus: int, ns_steps: int) -> bool:
     """Whether a group of ``count`` rows x cols matrices, run by itself, takes
     the direct path: where its estimate is a tenth below the staged path's (the
-    estimates' error is 6%, and the direct path's workspace is larger by X)."""
+    estimates' error is as large, and the direct path's workspace is larger by
+    X)."""
     m, n = min(rows, cols), max(rows, cols)
     return (_direct_fits(m, n, ns_steps)
             and _direct_us(((m, n, count),)) < 0.9 * _staged_us(m, n, count, cus))
@@ -432,6 +436,11 @@ def group_sizes(count: int, cap: int, m: int, n: int, cus: int) -> list[int]:
     number of matrices covered.  Tiles follow the library's choice for the
     group's size (``gemm_tile``), and a group on the 128 tile takes 256 x 256
     updates from m = 1024 when both padded edges are multiples of 256.
+
+    The model counts whole rounds; a last round of few 256-wide tiles costs
+    less, since it runs as 128-wide ones (launch_gemm).  Measured for 64 of
+    1024 x 4096: [24, 24, 16], its choice, 5842 us; [32, 32], whose 320
+    symmetric tiles are split after a round, 6006.
     """
     if count <= 0:
         return []
@@ -462,7 +471,8 @@ def group_sizes(count: int, cap: int, m: int, n: int, cus: int) -> list[int]:
 
 def _launch_rounds(tiles: int, tile: int, k: int, cus: int) -> float:
     """Time of one GEMM launch in k steps of a 256-wide tile: whole rounds of
-    the grid (two 128-wide workgroups per CU, a quarter of the work each)."""
+    the grid (two 128-wide workgroups per CU, a quarter of the work each); a
+    last round that runs split (launch_gemm) counts whole here."""
     slots = cus * (2 if tile == 128 else 1)
     return math.ceil(tiles / slots) * (k / 64) * (1.0 if tile == 256 else 0.5)
 
