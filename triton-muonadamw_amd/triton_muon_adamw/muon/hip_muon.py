@@ -212,7 +212,7 @@ def _check_bf16_2d(x: torch.Tensor, name: str) -> None:
         raise TypeError(f"{name} must be bfloat16 (got {x.dtype})")
 
 
-_PLAIN = (torch.Tensor, nn.Parameter, type(None))  # no attributes or copies of their own
+_PLAIN = (torch.Tensor, nn.Parameter)  # no attributes or copies of their own
 _NS_GRAM, _NS_POLY, _NS_UPDATE, _NS_STEP = range(4)  # MAMW_NS_*
 
 
@@ -262,7 +262,9 @@ def _ns_direct(op: int, X: torch.Tensor, S, out: torch.Tensor, a: float, b: floa
     autograd must refuse), an output with a forward-mode tangent (which the
     copy clears), 16-byte misaligned inputs (which it refuses unless it pads
     them), and sizes where it is the faster one."""
-    if any(type(t) not in _PLAIN for t in (X, S, out)) or forward_ad.unpack_dual(out).tangent is not None:
+    if type(X) not in _PLAIN or type(out) not in _PLAIN or S is not None and type(S) not in _PLAIN:
+        return False
+    if forward_ad._current_level >= 0 and forward_ad.unpack_dual(out).tangent is not None:
         return False
     m, n = X.shape
     shape = (m, m) if op in (_NS_GRAM, _NS_POLY) else (m, n)
