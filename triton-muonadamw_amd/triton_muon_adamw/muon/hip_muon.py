@@ -734,48 +734,53 @@ class HipMuon:
                     arr[i] = _lib.MuonMatrix(p.data_ptr(), p.grad.data_ptr(), self.momentum[p].data_ptr(), None,
                                              R, C, scaled_lr(self.lr, self.adjust_lr_fn, R, C), flags)
                 calls.append(_Call(dev, arr, len(chunk), 0, m, n, gi))
-        # The kernels: all of a device's concurrent classes direct or none, a
-        # class that runs by itself as it pays.
-        for dev in dict.fromkeys(c.device for c in calls):
-            cus = torch.cuda.get_device_properties(dev).multi_processor_count
-            mine = [c for c in calls if c.device == dev]
-            fits = {c: _direct_fits(c.m, c.n_, self.steps)
-                    and _direct_workspace_bytes(c.arr, c.n, self.steps) <= limits[dev] for c in mine}
-            together = (concurrent and all(fits.values())
-                        and direct_set_pays(tuple((c.m, c.n_, c.n) for c in mine), cus, self.steps,
-                                            len(_merge(mine, self.steps, limits[dev]))))
-            for c in mine:
-                c.direct = together if concurrent else fits[c] and direct_pays(c.m, c.n_, c.n, cus, self.steps)
-                c.ws_bytes = (_direct_workspace_bytes(c.arr, c.n, self.steps) if c.direct
-                              else _workspace_bytes(c.n, c.m, c.n_, self.steps))
-        # Concurrent classes, longest first (a class's own launches keep their
-        # order: stable sort), the staged ones on streams.  Direct ones need
-        # none: one launch on the caller's holds them all (up to
-        # MUON_DIRECT_MAX matrices).
-        self._lanes = {}
+        # The kernels: all of a device's concurrent classes direct or none (then
+        # as few launches as hold them), a class that runs by itself as it
+        # pays.  Concurrent classes longest first (a class's own launches keep
+        # their order: stable sort), the staged ones on streams.
+        def fits(c):
+            return (_direct_fits(c.m, c.n_, self.steps)
+                    and _direct_workspace_bytes(c.arr, c.n, self.steps) <= limits[c.device])
+
+        cus = {dev: torch.cuda.get_device_properties(dev).multi_processor_count for dev in limits}
         if concurrent:
-            cus = {c.device: torch.cuda.get_device_properties(c.device).multi_processor_count for c in calls}
-            self._lanes, times = _lanes([c for c in calls if not c.direct], self.steps, cus)
-            for key in {(c.device, c.group) for c in calls if c.direct}:
-                times[key] = _class_time(calls, key, self.steps, cus[key[0]])
+            times = {key: _class_time(calls, key, self.steps, cus[key[0]]) for key in {(c.device, c.group) for c in calls}}
             calls.sort(key=lambda c: -times[(c.device, c.group)])
-        launches, need = [], {}
-        for dev in dict.fromkeys(c.device for c in calls):
+        runs: list[list[_Call]] = []
+        for dev in limits:
             mine = [c for c in calls if c.device == dev]
-            merged = concurrent and mine[0].direct
-            for run in (_merge(mine, self.steps, limits[dev]) if merged else [[c] for c in mine]):
-                arr, n, wsb, lane, key = run[0].arr, run[0].n, run[0].ws_bytes, None, dev
-                if concurrent and not run[0].direct:
-                    lane, key = self._lanes[(dev, run[0].group)], (dev, run[0].group)
-                if len(run) > 1:
-                    arr, at = _entries(run), 0
-                    for c in run:  # the groups' entries are those of the launch
-                        c.arr = (_lib.MuonMatrix * c.n).from_buffer(arr, at * ctypes.sizeof(_lib.MuonMatrix))
-                        at += c.n
-                    n = at
-                    wsb = _direct_workspace_bytes(arr, n, self.steps)
-                need[key] = max(need.get(key, 0), wsb)
-                launches.append(_Launch(dev, arr, n, run[0].direct, lane, key))
+            if concurrent:
+                classes = tuple((c.m, c.n_, c.n) for c in mine)
+                direct = direct_set_pays(classes, cus[dev], self.steps) and all(fits(c) for c in mine)
+                if direct:
+                    merged = _merge(mine, self.steps, limits[dev])
+                    direct = direct_set_pays(classes, cus[dev], self.steps, len(merged))
+                for c in mine:
+                    c.direct = direct
+                runs += merged if direct else [[c] for c in mine]
+            else:
+                for c in mine:
+                    c.direct = direct_pays(c.m, c.n_, c.n, cus[dev], self.steps) and fits(c)
+                runs += [[c] for c in mine]
+        for c in calls:
+            c.ws_bytes = (_direct_workspace_bytes(c.arr, c.n, self.steps) if c.direct
+                          else _workspace_bytes(c.n, c.m, c.n_, self.steps))
+        self._lanes = _lanes([c for c in calls if not c.direct], self.steps, cus)[0] if concurrent else {}
+        launches, need = [], {}
+        for run in runs:
+            dev = run[0].device
+            arr, n, wsb, lane, key = run[0].arr, run[0].n, run[0].ws_bytes, None, dev
+            if concurrent and not run[0].direct:
+                lane, key = self._lanes[(dev, run[0].group)], (dev, run[0].group)
+            if len(run) > 1:
+                arr, at = _entries(run), 0
+                for c in run:  # the groups' entries are those of the launch
+                    c.arr = (_lib.MuonMatrix * c.n).from_buffer(arr, at * ctypes.sizeof(_lib.MuonMatrix))
+                    at += c.n
+                n = at
+                wsb = _direct_workspace_bytes(arr, n, self.steps)
+            need[key] = max(need.get(key, 0), wsb)
+            launches.append(_Launch(dev, arr, n, run[0].direct, lane, key))
         for key in [k for k in self._ws if k not in need]:
             del self._ws[key]
             self._ws_home.pop(key, None)
